@@ -149,7 +149,39 @@ struct GaugePassArgs {
   CsPoly poly;
 };
 
-// Deterministic block reduction: wavefront shuffles, then a fixed-order sum over the block's
+// Sum of v over the 64 lanes, in every lane, as the shuffle tree v[l] += v[l + 32], [l + 16], ... , [l + 1]
+// forms it in lane 0 (addition commutes, so each level adds the same pairs), by lane permutes of the vector
+// ALU: the two half and row swaps, then rotations within rows of 16.  A tree of LDS permutes (__shfl_down)
+// takes six dependent LDS round trips per value, which cost the update kernel and every workgroup
+// reduction 1-1.5 us.
+template <int CTRL> __device__ __forceinline__ double dpp_move(double v)
+{
+  const uint64_t b = __builtin_bit_cast(uint64_t, v);
+  const uint32_t lo = (uint32_t)__builtin_amdgcn_mov_dpp((int)(uint32_t)b, CTRL, 0xf, 0xf, true);
+  const uint32_t hi = (uint32_t)__builtin_amdgcn_mov_dpp((int)(uint32_t)(b >> 32), CTRL, 0xf, 0xf, true);
+  return __builtin_bit_cast(double, (uint64_t)lo | ((uint64_t)hi << 32));
+}
+__device__ __forceinline__ double wave_sum(double v)
+{
+  typedef uint32_t u2 __attribute__((ext_vector_type(2)));
+  uint64_t b = __builtin_bit_cast(uint64_t, v);
+  u2 lo = __builtin_amdgcn_permlane32_swap((uint32_t)b, (uint32_t)b, false, false);
+  u2 hi = __builtin_amdgcn_permlane32_swap((uint32_t)(b >> 32), (uint32_t)(b >> 32), false, false);
+  v = __builtin_bit_cast(double, (uint64_t)lo.x | ((uint64_t)hi.x << 32)) +
+      __builtin_bit_cast(double, (uint64_t)lo.y | ((uint64_t)hi.y << 32));
+  b = __builtin_bit_cast(uint64_t, v);
+  lo = __builtin_amdgcn_permlane16_swap((uint32_t)b, (uint32_t)b, false, false);
+  hi = __builtin_amdgcn_permlane16_swap((uint32_t)(b >> 32), (uint32_t)(b >> 32), false, false);
+  v = __builtin_bit_cast(double, (uint64_t)lo.x | ((uint64_t)hi.x << 32)) +
+      __builtin_bit_cast(double, (uint64_t)lo.y | ((uint64_t)hi.y << 32));
+  v += dpp_move<0x128>(v);  // row_ror:8
+  v += dpp_move<0x124>(v);
+  v += dpp_move<0x122>(v);
+  v += dpp_move<0x121>(v);
+  return v;
+}
+
+// Deterministic block reduction: wavefront sums, then a fixed-order sum over the block's
 // wavefronts; thread k < K writes slot k of the block's row.
 // Sum of v over a block of NTB threads, stored by threads 0..K-1 into row[0..K).
 template <int K, int NTB>
@@ -157,8 +189,7 @@ __device__ __forceinline__ void block_reduce_store_nt(double (&v)[K], double *ro
 {
   __shared__ double sh[NTB / 64][K];
 #pragma unroll
-  for (int k = 0; k < K; ++k)
-    for (int off = 32; off > 0; off >>= 1) v[k] += __shfl_down(v[k], off, 64);
+  for (int k = 0; k < K; ++k) v[k] = wave_sum(v[k]);
   const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
   if (lane == 0)
 #pragma unroll

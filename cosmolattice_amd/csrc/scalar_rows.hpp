@@ -172,8 +172,7 @@ __device__ __forceinline__ void block_reduce_rows(double (&v)[K], double *row)
 {
   __shared__ double sh[NW][K];
 #pragma unroll
-  for (int k = 0; k < K; ++k)
-    for (int off = 32; off > 0; off >>= 1) v[k] += __shfl_down(v[k], off, 64);
+  for (int k = 0; k < K; ++k) v[k] = wave_sum(v[k]);
   const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
   if (lane == 0)
 #pragma unroll

@@ -44,7 +44,7 @@ __device__ inline double sf_kernel(const clmi_background &b, const ModelConsts &
 
 // Fixed-order sum of `rows` partial rows by a block of NT threads: thread t adds rows t, t + NT, ... in
 // that order, four rows in flight per batch (each row one 64-byte line, read as four 16-byte loads),
-// then wavefront shuffles, then the wavefront sums in order.  Result in out[0..kNumRed)
+// then wavefront sums, then those in order.  Result in out[0..kNumRed)
 // (shared memory); ends with a barrier.  The rows are 64-byte aligned (kNumRed = 8 doubles).
 template <int NT>
 __device__ inline void sum_partials(const double *partials, int rows, double *out)
@@ -77,8 +77,7 @@ __device__ inline void sum_partials(const double *partials, int rows, double *ou
         }
   }
 #pragma unroll
-  for (int k = 0; k < kNumRed; ++k)
-    for (int off = 32; off > 0; off >>= 1) v[k] += __shfl_down(v[k], off, 64);
+  for (int k = 0; k < kNumRed; ++k) v[k] = wave_sum(v[k]);
   if ((t & 63) == 0)
 #pragma unroll
     for (int k = 0; k < kNumRed; ++k) sh[t >> 6][k] = v[k];
