@@ -29,6 +29,13 @@ HIP_SOURCES = [
     "scalar_rows_f64.hip",
     "scalar_rows_f64_1f.hip",
     "scalar_rows_batch.hip",
+    "scalar_resident.hip",
+    "scalar_resident_lf_f64.hip",
+    "scalar_resident_lf_f32.hip",
+    "scalar_resident_vv_f64.hip",
+    "scalar_resident_vv_f32.hip",
+    "scalar_resident_pv_f64.hip",
+    "scalar_resident_pv_f32.hip",
     "gauge_pass.hip",
     "gauge_tiled.hip",
     "background.hip",

@@ -13,6 +13,7 @@
 #include <hipfft/hipfft.h>
 
 #include <algorithm>
+#include <climits>
 #include <cstddef>
 #include <cmath>
 #include <cstring>
@@ -61,6 +62,14 @@ struct clmi_ctx {
   ScalarPoly spoly{};
   CsPoly cpoly{};
   ModelConsts mc{};
+
+  // resident evolver of small scalar-singlet lattices (its buffers are allocated at the first use)
+  bool resident = false;
+  ResidentPlan resp;
+  uint64_t *res_lines = nullptr;
+  void *res_xch = nullptr;
+  int *res_err = nullptr;  // page-locked, device-visible
+  uint32_t res_epoch = 0;
 
   bool synced = true;
   bool pending_drift = false;
@@ -186,6 +195,16 @@ int prof_event(clmi_ctx *c)
   }
   HIPCHK(c, hipEventRecord(c->ev[c->ev_used], c->stream));
   c->ev_used++;
+  return CLMI_OK;
+}
+
+// Wait for the stream, then report a resident evolver whose workgroups lost each other (its launch leaves the
+// arrays it read untouched and writes no result).
+int sync_stream(clmi_ctx *c)
+{
+  HIPCHK(c, hipStreamSynchronize(c->stream));
+  if (c->res_err && __atomic_load_n(c->res_err, __ATOMIC_RELAXED) != 0)
+    return fail(c, CLMI_E_HIP, "the resident evolver's workgroups timed out waiting for each other");
   return CLMI_OK;
 }
 
@@ -346,6 +365,69 @@ bool double_kick_ok(const clmi_ctx *c)
   return (c->rowk || c->tiled) && c->cfg.n_scalars > 0 && c->cfg.n_cscalars == 0 && !(c->cfg.flags & CLMI_FLAG_NO_DOUBLE_KICK);
 }
 
+// Fewest passes that the resident evolver takes: a cooperative launch with its load and store of the state costs
+// 25-47 us and saves 8-20 us a pass, so it pays from 3 to 4 passes on (64^3 one field FP64: 25 us, 6.0 against
+// 15 us a pass; 128^3 two fields FP64: 47 us, 17.7 against 37 us).
+constexpr int kResMinPasses = 4;
+
+// Runs `passes` passes of a scheme as one launch of the resident evolver, where the lattice has a plan for it:
+// drift + kick passes (RES_LF), double-kick passes (RES_VV) or pairs of drift + kick and drift (RES_PV).
+// *done = false: not taken (nothing was changed), the caller runs the passes one by one, which gives the
+// same bits.  Not taken: too few passes for the cooperative launch to pay, pass timing on, a background snapshot
+// asked for, more weights than its arguments hold, no memory for its buffers, or a device too small for its tiles.
+int run_resident(clmi_ctx *c, int scheme, int passes, const double *ws, int nws, bool *done)
+{
+  *done = false;
+  if (!c->resident || passes < kResMinPasses || c->prof || c->snap || nws > kResMaxWeights) return CLMI_OK;
+  const int nf = c->cfg.n_scalars;
+  const size_t tiles = (size_t)c->resp.groups * c->resp.chunks;
+  const size_t line_bytes = 2 * tiles * 8 * sizeof(uint64_t);
+  if (!c->res_lines) {
+    const size_t xb = 2 * (size_t)nf * c->V * bytes_field(c->f32);
+    if (hipMalloc(&c->res_lines, line_bytes) != hipSuccess || hipMalloc(&c->res_xch, xb) != hipSuccess ||
+        hipHostMalloc((void **)&c->res_err, sizeof(int), hipHostMallocMapped) != hipSuccess) {
+      (void)hipGetLastError();
+      c->resident = false;  // a small lattice that cannot have them runs pass by pass
+      if (c->res_lines) (void)hipFree(c->res_lines);
+      if (c->res_xch) (void)hipFree(c->res_xch);
+      c->res_lines = nullptr;
+      c->res_xch = nullptr;
+      return CLMI_OK;
+    }
+    *c->res_err = 0;
+    c->res_epoch = UINT32_MAX;  // clears the lines below
+  }
+  if (UINT32_MAX - c->res_epoch <= (uint32_t)passes) {
+    HIPCHK(c, hipMemsetAsync(c->res_lines, 0, line_bytes, c->stream));
+    c->res_epoch = 0;
+  }
+  ResidentArgs r{};
+  r.a = scalar_args(c, c->cur_fS, 1 - c->cur_fS, c->cur_pS, 1 - c->cur_pS, 0.0, 0.0, 0);
+  r.st = c->dstate;
+  r.mc = c->mc;
+  r.passes = passes;
+  r.nws = nws;
+  for (int i = 0; i < nws; ++i) r.ws[i] = ws[i];
+  r.groups = c->resp.groups;
+  r.chunks = c->resp.chunks;
+  r.lines = c->res_lines;
+  r.xch = c->res_xch;
+  r.epoch0 = c->res_epoch;
+  r.err = c->res_err;
+  const hipError_t e = launch_scalar_resident(scheme, nf, c->f32, poly_kind(c->spoly, nf), c->resp, r, c->stream);
+  if (e == hipErrorCooperativeLaunchTooLarge) {
+    (void)hipGetLastError();
+    c->resident = false;
+    return CLMI_OK;
+  }
+  HIPCHK(c, e);
+  c->res_epoch += (uint32_t)passes;
+  c->cur_fS = 1 - c->cur_fS;
+  c->cur_pS = 1 - c->cur_pS;
+  *done = true;
+  return CLMI_OK;
+}
+
 // Apply the deferred drift of the last leapfrog step (drift-only pass + storeFieldsAverages).
 int flush(clmi_ctx *c)
 {
@@ -421,7 +503,7 @@ int ensure_fft(clmi_ctx *c, bool r2c, bool c2r, bool two)
 int read_state(clmi_ctx *c, DevState *h)
 {
   HIPCHK(c, hipMemcpyAsync(h, c->dstate, sizeof(DevState), hipMemcpyDeviceToHost, c->stream));
-  HIPCHK(c, hipStreamSynchronize(c->stream));
+  CHK(sync_stream(c));
   return CLMI_OK;
 }
 
@@ -536,6 +618,15 @@ int clmi_create(const clmi_config *cfg, clmi_ctx **out)
       c->rows_g = grows_t;
     }
   }
+  // The resident evolver: integer alpha (its background update has no general power), a CU for every tile (the
+  // launch itself checks that they fit).
+  if (!(g.flags & (CLMI_FLAG_NO_TILED | CLMI_FLAG_NO_DOUBLE_KICK)) && g.n_cscalars == 0 && g.N % 64 == 0 &&
+      g.alpha == std::rint(g.alpha) && std::fabs(g.alpha) <= 15.0 && resident_plan(g.N, g.n_scalars, &c->resp)) {
+    int cus = 0, coop = 0;
+    c->resident = hipDeviceGetAttribute(&cus, hipDeviceAttributeMultiprocessorCount, c->device) == hipSuccess &&
+                  hipDeviceGetAttribute(&coop, hipDeviceAttributeCooperativeLaunch, c->device) == hipSuccess && coop &&
+                  cus >= c->resp.groups * c->resp.chunks;
+  }
   // Partial-sum rows: a reducing step pass writes the scalar sector's rows, then the charged-scalar + U(1)
   // sector's after them; the measurement kernels write at most kMaxPassBlocks rows each.
   const size_t srows = g.n_scalars == 0 ? 0
@@ -606,6 +697,9 @@ void clmi_destroy(clmi_ctx *c)
     }
   if (c->partials) (void)hipFree(c->partials);
   if (c->dscratch) (void)hipFree(c->dscratch);
+  if (c->res_lines) (void)hipFree(c->res_lines);
+  if (c->res_xch) (void)hipFree(c->res_xch);
+  if (c->res_err) (void)hipHostFree(c->res_err);
   if (c->dstate) (void)hipFree(c->dstate);
   if (c->stage) (void)hipFree(c->stage);
   if (c->fk) (void)hipFree(c->fk);
@@ -624,7 +718,7 @@ const char *clmi_last_error(const clmi_ctx *c) { return c ? c->err.c_str() : g_c
 int clmi_synchronize(clmi_ctx *c)
 {
   CHK(check_ctx(c));
-  HIPCHK(c, hipStreamSynchronize(c->stream));
+  CHK(sync_stream(c));
   return CLMI_OK;
 }
 
@@ -647,7 +741,7 @@ int clmi_upload_field(clmi_ctx *c, int kind, int index, int comp, const double *
     else
       HIPCHK(c, launch_to_f32(c->stage, (float *)a->p, c->V, c->stream));
   }
-  HIPCHK(c, hipStreamSynchronize(c->stream));
+  CHK(sync_stream(c));
   return CLMI_OK;
 }
 
@@ -667,7 +761,7 @@ int clmi_download_field(clmi_ctx *c, int kind, int index, int comp, double *host
     HIPCHK(c, launch_join_f64((const float *)a->p, a->lo, c->stage, c->V, c->stream));
     HIPCHK(c, hipMemcpyAsync(host, c->stage, n * sizeof(double), hipMemcpyDeviceToHost, c->stream));
   }
-  HIPCHK(c, hipStreamSynchronize(c->stream));
+  CHK(sync_stream(c));
   return CLMI_OK;
 }
 
@@ -681,7 +775,7 @@ int clmi_set_background(clmi_ctx *c, const clmi_background *bg)
   h.bg = *bg;
   HIPCHK(c, hipMemcpyAsync(c->dstate, &h, sizeof(DevState), hipMemcpyHostToDevice, c->stream));
   CHK(update(c, 0, {}));
-  HIPCHK(c, hipStreamSynchronize(c->stream));
+  CHK(sync_stream(c));
   return CLMI_OK;
 }
 
@@ -702,7 +796,7 @@ int clmi_lf_init(clmi_ctx *c, int restart)
   CHK(flush(c));
   c->synced = restart == 0;
   if (c->synced && c->cfg.expansion) CHK(update(c, 0, {{OP_LF_INIT, 0.0}}));
-  HIPCHK(c, hipStreamSynchronize(c->stream));
+  CHK(sync_stream(c));
   return CLMI_OK;
 }
 
@@ -713,6 +807,12 @@ int clmi_lf_evolve(clmi_ctx *c, int nsteps)
   const bool ex = c->cfg.expansion != 0;
   const double dt = c->cfg.dt;
   for (int n = 0; n < nsteps; ++n) {
+    if (c->pending_drift && !c->synced) {
+      // every remaining step is the same drift + kick pass
+      bool done = false;
+      CHK(run_resident(c, RES_LF, nsteps - n, nullptr, 0, &done));
+      if (done) return CLMI_OK;
+    }
     const double w = c->synced ? 0.5 : 1.0;
     if (c->pending_drift) {
       CHK(pass_update(c, true, true, ex, dt, w * dt, w * dt, ex, {{OP_STORE_FIELDS, 0.0}, {OP_LF_MOMENTA, 0.0}}));
@@ -760,7 +860,9 @@ int clmi_vv_evolve(clmi_ctx *c, const double *ws, int nws, int nsteps)
       CHK(pass_update(c, false, true, ex, 0.0, wk(0) * dt / 2, dt / 2 * wk(0), ex,
                       {{OP_VV_MOMENTA, 0.0}, {OP_VV_DRIFT_SF, wk(0)}}));
     }
-    for (int k = 0; k < K; ++k) {
+    bool done = false;
+    CHK(run_resident(c, RES_VV, K - 1, ws, nws, &done));
+    for (int k = done ? K - 1 : 0; k < K; ++k) {
       const double w = wk(k);
       if (k + 1 < K) {
         const double w2 = wk(k + 1);
@@ -807,12 +909,15 @@ int clmi_pv_evolve(clmi_ctx *c, const double *ws, int nws, int nsteps)
   const int stages = (nws - 1) * 2 + 1;
   auto weight = [&](int s) { return ws[s < nws ? s : stages - s - 1]; };
   if (!ex) CHK(update(c, 0, {{OP_PV_DRIFT_AI, 0.0}}));
-  for (int n = 0; n < nsteps; ++n)
+  if (ex && nsteps > 0) CHK(update(c, 0, {{OP_PV_SF_FIRST, weight(0)}}));
+  bool done = false;
+  if (nsteps <= INT_MAX / (2 * stages))
+    CHK(run_resident(c, RES_PV, 2 * nsteps * stages, ws, nws, &done));
+  for (int n = 0; n < nsteps && !done; ++n)
     for (int s = 0; s < stages; ++s) {
       const double w = weight(s);
       // drift (aI of the stage start) + kick (half-step aI) in one pass, then the mid-stage update; the
       // stage's first scale-factor drift rides on the previous stage's last update after the first stage
-      if (ex && n == 0 && s == 0) CHK(update(c, 0, {{OP_PV_SF_FIRST, w}}));
       CHK(pass_update(c, true, true, ex, dt / 2 * w, w * dt, w * dt, ex, {{OP_PV_MID, w}}));
       // second drift (new aI) + storeFieldsAveragesInt
       const bool last = n == nsteps - 1 && s == stages - 1;
@@ -851,7 +956,7 @@ int clmi_set_all_averages(clmi_ctx *c)
   CHK(check_ctx(c));
   CHK(flush(c));
   CHK(pass_update(c, false, false, true, 0.0, 0.0, 0.0, true, {{OP_SET_ALL, 0.0}}));
-  HIPCHK(c, hipStreamSynchronize(c->stream));
+  CHK(sync_stream(c));
   return CLMI_OK;
 }
 
@@ -937,7 +1042,7 @@ int clmi_gauss_u1(clmi_ctx *c, double out[3])
   HIPCHK(c, launch_sum_rows(c->partials, gblocks, c->dscratch, c->stream));
   double h[kNumRed];
   HIPCHK(c, hipMemcpyAsync(h, c->dscratch, sizeof(h), hipMemcpyDeviceToHost, c->stream));
-  HIPCHK(c, hipStreamSynchronize(c->stream));
+  CHK(sync_stream(c));
   const double V = (double)c->V;
   out[0] = (h[0] / V) / (h[1] / V);
   out[1] = h[3] / V;
@@ -967,7 +1072,7 @@ int clmi_field_means(clmi_ctx *c, int kind, int index, int comp, double scale, d
   HIPCHK(c, launch_sum_rows(c->partials, blocks, c->dscratch, c->stream));
   double h[kNumRed];
   HIPCHK(c, hipMemcpyAsync(h, c->dscratch, sizeof(h), hipMemcpyDeviceToHost, c->stream));
-  HIPCHK(c, hipStreamSynchronize(c->stream));
+  CHK(sync_stream(c));
   out[0] = h[0] / (double)c->V;
   out[1] = h[1] / (double)c->V;
   return CLMI_OK;
@@ -995,7 +1100,7 @@ int clmi_field_stats(clmi_ctx *c, int kind, int index, int comp, double out[3])
   HIPCHK(c, launch_sum_rows(c->partials, blocks, c->dscratch, c->stream));
   double h[kNumRed];
   HIPCHK(c, hipMemcpyAsync(h, c->dscratch, sizeof(h), hipMemcpyDeviceToHost, c->stream));
-  HIPCHK(c, hipStreamSynchronize(c->stream));
+  CHK(sync_stream(c));
   const double dx = c->cfg.dx;
   out[0] = h[0] / (double)c->V;
   out[1] = h[1] / (double)c->V;
@@ -1053,7 +1158,7 @@ int clmi_norm_averages(clmi_ctx *c, int kind, int index, double out[2])
   HIPCHK(c, launch_sum_rows(c->partials, blocks, c->dscratch, c->stream));
   double h[kNumRed];
   HIPCHK(c, hipMemcpyAsync(h, c->dscratch, sizeof(h), hipMemcpyDeviceToHost, c->stream));
-  HIPCHK(c, hipStreamSynchronize(c->stream));
+  CHK(sync_stream(c));
   out[0] = h[0] / (double)c->V;
   out[1] = h[1] / (double)c->V;
   return CLMI_OK;
@@ -1080,7 +1185,7 @@ int clmi_monomial_averages(clmi_ctx *c, double *out)
   HIPCHK(c, launch_sum_rows(c->partials, blocks, c->dscratch, c->stream));
   double h[kNumRed];
   HIPCHK(c, hipMemcpyAsync(h, c->dscratch, sizeof(h), hipMemcpyDeviceToHost, c->stream));
-  HIPCHK(c, hipStreamSynchronize(c->stream));
+  CHK(sync_stream(c));
   for (int t = 0; t < c->spoly.nterms; ++t) out[t] = h[t] / (double)c->V;
   return CLMI_OK;
 }
@@ -1127,7 +1232,7 @@ int clmi_spectrum_bins_npow(clmi_ctx *c, int kind, int index, int comp, double d
   }
   FFTCHK(c, hipfftExecD2Z(c->plan_r2c, (hipfftDoubleReal *)fft_in, (hipfftDoubleComplex *)c->fk));
   if (c->bins.nbins != nbins || c->bins.dk != dk || c->bins.N != c->N) {
-    HIPCHK(c, hipStreamSynchronize(c->stream));
+    CHK(sync_stream(c));
     HIPCHK(c, build_bin_table(c->bins, c->N, dk, nbins));
   }
   if (c->bin_out_n < nbins) {
@@ -1139,7 +1244,7 @@ int clmi_spectrum_bins_npow(clmi_ctx *c, int kind, int index, int comp, double d
   }
   HIPCHK(c, launch_bin_sums(c->bins, c->fk, c->bin_out, c->stream, npow));
   HIPCHK(c, hipMemcpyAsync(sum_f2, c->bin_out, sizeof(double) * nbins, hipMemcpyDeviceToHost, c->stream));
-  HIPCHK(c, hipStreamSynchronize(c->stream));
+  CHK(sync_stream(c));
   for (int b = 0; b < nbins; ++b) {
     if (count) count[b] = c->bins.count[b];
     if (mean_n) mean_n[b] = c->bins.mean_n[b];
@@ -1192,7 +1297,7 @@ int clmi_grf_scalar(clmi_ctx *c, int index, uint64_t seed, uint32_t stream, doub
   HIPCHK(c, launch_grf_finish(c->stage, scale, fld0, f.p, f.lo, c->f32, c->V, c->stream));
   FFTCHK(c, hipfftExecZ2D(c->plan_c2r, (hipfftDoubleComplex *)c->fk2, (hipfftDoubleReal *)c->stage));
   HIPCHK(c, launch_grf_finish(c->stage, scale, pi0, p.p, nullptr, c->f32, c->V, c->stream));
-  HIPCHK(c, hipStreamSynchronize(c->stream));
+  CHK(sync_stream(c));
   return CLMI_OK;
 }
 
@@ -1252,7 +1357,7 @@ int clmi_grf_u1(clmi_ctx *c, uint64_t seed, uint32_t stream, const double mass2[
       HIPCHK(c, launch_grf_finish(c->stage, scale, 0.0, P.p, nullptr, c->f32, c->V, c->stream));
     }
   }
-  HIPCHK(c, hipStreamSynchronize(c->stream));
+  CHK(sync_stream(c));
   return CLMI_OK;
 }
 
@@ -1388,7 +1493,7 @@ struct AdjRun {
 int adj_read_red(clmi_ctx *c, const AdjRun &r, double out[kAdjRed])
 {
   HIPCHK(c, hipMemcpyAsync(out, r.red, sizeof(double) * kAdjRed, hipMemcpyDeviceToHost, c->stream));
-  HIPCHK(c, hipStreamSynchronize(c->stream));
+  CHK(sync_stream(c));
   return CLMI_OK;
 }
 
@@ -1472,7 +1577,7 @@ int clmi_adjoint_lf(clmi_ctx *c, int nsteps, int checkpoint_every, int bg_from_f
   c->snap = nullptr;
   HIPCHK(c, hipMemcpyAsync(tape.data(), run.tape, sizeof(clmi_background) * (size_t)(nsteps + 1),
                            hipMemcpyDeviceToHost, c->stream));
-  HIPCHK(c, hipStreamSynchronize(c->stream));
+  CHK(sync_stream(c));
   if (!ex) {
     for (int n = 1; n <= nsteps; ++n) tape[n] = tape[0];
     HIPCHK(c, hipMemcpyAsync(run.tape, tape.data(), sizeof(clmi_background) * (size_t)(nsteps + 1),
@@ -1538,7 +1643,7 @@ int clmi_adjoint_lf(clmi_ctx *c, int nsteps, int checkpoint_every, int bg_from_f
     h.lam_U = lam_U;
     for (int t = 0; t < nt; ++t) h.gc[t] = gc[t];
     HIPCHK(c, hipMemcpyAsync(run.sc, &h, sizeof(AdjScalars), hipMemcpyHostToDevice, c->stream));
-    HIPCHK(c, hipStreamSynchronize(c->stream));
+    CHK(sync_stream(c));
   }
   // Per reverse step n: the pi transpose of step n, then one pass with the kick transpose of step n
   // fused with the fields transpose of state n (which the original order runs first thing in step
@@ -1602,7 +1707,7 @@ int clmi_adjoint_lf(clmi_ctx *c, int nsteps, int checkpoint_every, int bg_from_f
   {
     AdjScalars h{};
     HIPCHK(c, hipMemcpyAsync(&h, run.sc, sizeof(AdjScalars), hipMemcpyDeviceToHost, c->stream));
-    HIPCHK(c, hipStreamSynchronize(c->stream));
+    CHK(sync_stream(c));
     lam_aI = h.lam_aI;
     lam_aDotSI = h.lam_aDotSI;
     lam_pi2SI = h.lam_pi2SI;
@@ -1654,7 +1759,7 @@ int clmi_adjoint_lf(clmi_ctx *c, int nsteps, int checkpoint_every, int bg_from_f
   CHK(clmi_set_background(c, &b_fin));
   c->synced = true;
   c->pending_drift = false;
-  HIPCHK(c, hipStreamSynchronize(c->stream));
+  CHK(sync_stream(c));
   return CLMI_OK;
 }
 
@@ -2166,6 +2271,9 @@ int clmi_plan_report(const clmi_ctx *c, char *report, size_t report_len)
              "\n";
     else
       rep += "k_scalar_pass\n";
+    if (c->resident)
+      rep += "k_scalar_resident VZ=" + std::to_string(c->resp.VZ) + " P=" + std::to_string(c->resp.P) +
+             " tiles=" + std::to_string(c->resp.groups * c->resp.chunks) + "\n";
   }
   if (c->cfg.n_cscalars > 0) {
     if (c->gtiled)

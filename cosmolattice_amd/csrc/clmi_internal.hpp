@@ -236,6 +236,33 @@ struct UpdMember {    // one lattice's background update inside a batched launch
 };
 hipError_t launch_update_batch(const UpdMember *d_members, int n, const UpdateOps &ops, hipStream_t s);
 
+// ---- resident evolver of small lattices (scalar_resident.hpp) ----
+constexpr int kResThreads = 512;
+constexpr int kResMaxWeights = 16;  // composition weights
+enum ResScheme : int { RES_LF = 0, RES_VV = 1, RES_PV = 2 };
+struct ResidentArgs {
+  ScalarPassArgs a;  // current arrays (in) and where the final ones go (out); a.cdt, a.ckick unused
+  DevState *st;
+  ModelConsts mc;
+  int passes;
+  int nws;
+  double ws[kResMaxWeights];
+  int groups, chunks;  // tiles along x and within a plane
+  uint64_t *lines;     // 2 x 8 x tiles words: partial sums with the epoch of their pass
+  void *xch;           // 2 x n_scalars x V momenta: boundary values of the last two kicks
+  uint32_t epoch0;     // passes of earlier launches on these buffers
+  int pad;
+  int *err;            // host-visible: a wait between workgroups ran out
+};
+// Tiles of the resident evolver for an N^3 lattice: chunks of kResThreads * VZ sites of a plane by P planes.
+struct ResidentPlan {
+  int VZ = 0, P = 0, groups = 0, chunks = 0;
+  bool ragged = false;  // tiles that are not full
+};
+bool resident_plan(int N, int nf, ResidentPlan *p);
+// hipErrorCooperativeLaunchTooLarge where the device does not hold all tiles at once.
+hipError_t launch_scalar_resident(int scheme, int nf, bool f32, int pk, const ResidentPlan &p, const ResidentArgs &r, hipStream_t s);
+
 // ---- adjoint (adjoint_kernels.hip) ----
 constexpr int kAdjRed = 32;  // partial-sum slots of the adjoint reductions
 constexpr int kAdjMaxRows = 1024;  // partial rows (one per workgroup) of an adjoint lattice kernel

@@ -1,0 +1,54 @@
+// Plan and launch of the resident evolver (kernel in scalar_resident.hpp).
+#include "clmi_internal.hpp"
+
+namespace clmi {
+
+const void *resident_kernel_lf_f64(int nf, const ResidentPlan &p, int pk);
+const void *resident_kernel_lf_f32(int nf, const ResidentPlan &p, int pk);
+const void *resident_kernel_vv_f64(int nf, const ResidentPlan &p, int pk);
+const void *resident_kernel_vv_f32(int nf, const ResidentPlan &p, int pk);
+const void *resident_kernel_pv_f64(int nf, const ResidentPlan &p, int pk);
+const void *resident_kernel_pv_f32(int nf, const ResidentPlan &p, int pk);
+
+namespace {
+const void *kernel_of(int scheme, int nf, bool f32, int pk, const ResidentPlan &p)
+{
+  if (nf < 1 || nf > 2) return nullptr;
+  switch (scheme) {
+    case RES_LF: return f32 ? resident_kernel_lf_f32(nf, p, pk) : resident_kernel_lf_f64(nf, p, pk);
+    case RES_VV: return f32 ? resident_kernel_vv_f32(nf, p, pk) : resident_kernel_vv_f64(nf, p, pk);
+    case RES_PV: return f32 ? resident_kernel_pv_f32(nf, p, pk) : resident_kernel_pv_f64(nf, p, pk);
+    default: return nullptr;
+  }
+}
+}  // namespace
+
+// One site per lane up to 64^3, two above (64 and 128 as the full-row pass has them).  Four planes per tile
+// where that gives at most 256 tiles -- one per CU, and half the sites per wave of eight-plane tiles --
+// else eight; 64^3 and 128^3 take eight, the full-row pass's group, so that their sums are the same.
+bool resident_plan(int N, int nf, ResidentPlan *p)
+{
+  if (nf < 1 || nf > 2 || N < 24 || N > 128 || (N & 1)) return false;
+  p->VZ = N <= 64 ? 1 : 2;
+  const int C = kResThreads * p->VZ;
+  p->chunks = (N * N + C - 1) / C;
+  for (int P : {4, 8}) {
+    p->P = P;
+    p->groups = (N + P - 1) / P;
+    if (N % 64 != 0 && p->groups * p->chunks <= 256) break;
+  }
+  p->ragged = N % p->P != 0 || (N * N) % C != 0;
+  return p->groups * p->chunks <= 256;
+}
+
+hipError_t launch_scalar_resident(int scheme, int nf, bool f32, int pk, const ResidentPlan &p, const ResidentArgs &r,
+                                  hipStream_t s)
+{
+  const void *k = kernel_of(scheme, nf, f32, pk, p);
+  if (!k || r.groups != p.groups || r.chunks != p.chunks || r.passes < 1) return hipErrorInvalidValue;
+  ResidentArgs args = r;
+  void *params[] = {&args};
+  return hipLaunchCooperativeKernel(k, dim3(p.groups * p.chunks), dim3(kResThreads), params, 0, s);
+}
+
+}  // namespace clmi

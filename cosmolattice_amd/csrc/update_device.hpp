@@ -9,9 +9,25 @@
 
 namespace clmi {
 
+// rpow(); INT: the exponent is known to be an integer of magnitude at most 32 (integer alpha), so the general
+// pow(), which costs a kernel that keeps its state in registers about 100 of them, is not compiled in.
+template <bool INT> __device__ __forceinline__ double bg_pow(double a, double e)
+{
+  if constexpr (!INT) return rpow(a, e);
+  int n = (int)fabs(e);
+  double p = 1.0, q = a;
+  while (n) {
+    if (n & 1) p *= q;
+    q *= q;
+    n >>= 1;
+  }
+  return e < 0 ? 1.0 / p : p;
+}
+
 // The scale-factor kernel of ScaleFactorKernels::get/getSI (evolvers/kernels/scalefactorkernels.h:27-124)
 // with the energy normalisations of definitions/energies.h:37-85, from the given volume averages.
-__device__ inline double sf_kernel_of(double a, double pi2S, double grad2S, double pi2CS, double grad2CS,
+template <bool INT>
+__device__ __forceinline__ double sf_kernel_of(double a, double pi2S, double grad2S, double pi2CS, double grad2CS,
                                       double pi2U1, double mag2U1, double pot, const ModelConsts &mc)
 {
   // a^-2, a^-4, a^-6 from one division (a serial chain on the updating thread)
@@ -31,15 +47,16 @@ __device__ inline double sf_kernel_of(double a, double pi2S, double grad2S, doub
     Emag = 0.5 * w2 * ia4 * mag2U1;
   }
   const double fm = mc.fStar / mc.MPl;
-  return rpow(a, 2 * mc.alpha + 1) / 3.0 * (fm * fm) *
+  return bg_pow<INT>(a, 2 * mc.alpha + 1) / 3.0 * (fm * fm) *
          ((mc.alpha - 2) * (Eks + Ekcs) + mc.alpha * (Egs + Egcs) + (mc.alpha - 1) * (Eel + Emag) +
           (mc.alpha + 1) * pot);
 }
 
 // ScaleFactorKernels::get: integer-time averages.
-__device__ inline double sf_kernel(const clmi_background &b, const ModelConsts &mc)
+template <bool INT>
+__device__ __forceinline__ double sf_kernel(const clmi_background &b, const ModelConsts &mc)
 {
-  return sf_kernel_of(b.aI, b.pi2AvI, b.grad2AvI, b.CSpi2AvI, b.CSgrad2AvI, b.U1pi2AvI, b.U1Mag2AvI, b.potAvI, mc);
+  return sf_kernel_of<INT>(b.aI, b.pi2AvI, b.grad2AvI, b.CSpi2AvI, b.CSgrad2AvI, b.U1pi2AvI, b.U1Mag2AvI, b.potAvI, mc);
 }
 
 // Fixed-order sum of `rows` partial rows by a block of NT threads: thread t adds rows t, t + NT, ... in
@@ -90,144 +107,160 @@ __device__ inline void sum_partials(const double *partials, int rows, double *ou
   __syncthreads();
 }
 
-// Executed by one thread.  red: finished volume averages (sums / N^3) of the last pass.
-__device__ inline void apply_update(DevState *st, const double *red, const ModelConsts &mc, const UpdateOps &ops)
+// One background operation (UpdateOp), executed by one thread.  red: finished volume averages (sums / N^3) of
+// the last pass.  a_drift > 0: the drift coefficients use this scale factor instead of aSI.
+template <bool INT>
+__device__ __forceinline__ void apply_op(DevState *st, const double *red, const ModelConsts &mc, const int op,
+                                         const double w, double &a_drift)
 {
   clmi_background &b = st->bg;
   const double dt = mc.dt;
-  double a_drift = -1.0;  // > 0: the drift coefficients use this scale factor instead of aSI
-  for (int o = 0; o < ops.n; ++o) {
-    const double w = ops.w[o];
-    switch (ops.op[o]) {
-      case OP_STORE_FIELDS:  // leapfrog.h:269-277
-        if (mc.ns > 0) b.grad2AvI = red[RED_GRAD2S];
-        if (mc.ncs > 0) b.CSgrad2AvI = red[RED_GRAD2CS];
-        if (mc.nu1 > 0) b.U1Mag2AvI = red[RED_B2U1];
-        b.potAvI = red[RED_POT];
-        break;
-      case OP_LF_MOMENTA:  // leapfrog.h:239-267 then 124-129 and 168-184
-        if (mc.ns > 0) {
-          b.pi2AvSIM = b.pi2AvSI;
-          b.pi2AvSI = red[RED_PI2S];
-          b.pi2AvI = 0.5 * (b.pi2AvSIM + b.pi2AvSI);
-        }
-        if (mc.ncs > 0) {
-          b.CSpi2AvSIM = b.CSpi2AvSI;
-          b.CSpi2AvSI = red[RED_PI2CS];
-          b.CSpi2AvI = 0.5 * (b.CSpi2AvSIM + b.CSpi2AvSI);
-        }
-        if (mc.nu1 > 0) {
-          b.U1pi2AvSIM = b.U1pi2AvSI;
-          b.U1pi2AvSI = red[RED_PI2U1];
-          b.U1pi2AvI = 0.5 * (b.U1pi2AvSIM + b.U1pi2AvSI);
-        }
-        st->K = sf_kernel(b, mc);
-        b.aDotSIM = b.aDotSI;
-        b.aDotSI += dt * st->K;
-        b.aDotI = (b.aDotSIM + b.aDotSI) / 2.0;
-        b.aIM = b.aI;
-        b.aI += dt * b.aDotSI;
-        b.aSI = (b.aIM + b.aI) / 2.0;
-        break;
-      case OP_LF_SYNC:  // leapfrog.h:105-112
-        if (mc.ns > 0) b.pi2AvI = red[RED_PI2S];
-        if (mc.ncs > 0) b.CSpi2AvI = red[RED_PI2CS];
-        if (mc.nu1 > 0) b.U1pi2AvI = red[RED_PI2U1];
-        st->K = sf_kernel(b, mc);
-        b.aDotI = b.aDotSI + dt / 2.0 * st->K;
-        break;
-      case OP_LF_INIT:  // leapfrog.h:35
-        st->K = sf_kernel(b, mc);
-        b.aDotSI = b.aDotI - dt / 2.0 * st->K;
-        break;
-      case OP_VV_SF_HALF:  // velocityverlet.h:165-168
-        st->K = sf_kernel(b, mc);
-        b.aDotSI = b.aDotI + (dt / 2) * st->K * w;
-        break;
-      case OP_VV_MOMENTA:  // velocityverlet.h:249-256
-        if (mc.ns > 0) b.pi2AvI = red[RED_PI2S];
-        if (mc.ncs > 0) b.CSpi2AvI = red[RED_PI2CS];
-        if (mc.nu1 > 0) b.U1pi2AvI = red[RED_PI2U1];
-        break;
-      case OP_VV_MOMENTA_KICK2:  // velocityverlet.h:249-256, scalar singlets only
-        b.pi2AvI = red[RED_PI2S_KICK2];
-        break;
-      case OP_VV_DRIFT_SF:  // velocityverlet.h:239-242
-        b.aIM = b.aI;
-        b.aI += dt * b.aDotSI * w;
-        b.aSI = (b.aIM + b.aI) / 2.0;
-        break;
-      case OP_VV_SF_ONE:  // velocityverlet.h:171-174
-        st->K = sf_kernel(b, mc);
-        b.aDotI = b.aDotSI + (dt / 2) * st->K * w;
-        break;
-      case OP_SET_ALL:  // averages.h:86-116
-        b.potAvI = red[RED_POT];
-        b.potAvSI = b.potAvI;
-        if (mc.ns > 0) {
-          b.pi2AvI = red[RED_PI2S];
-          b.pi2AvSI = b.pi2AvI;
-          b.grad2AvI = red[RED_GRAD2S];
-        }
-        if (mc.nu1 > 0) {
-          b.U1pi2AvI = red[RED_PI2U1];
-          b.U1pi2AvSI = b.U1pi2AvI;
-          b.U1Mag2AvI = red[RED_B2U1];
-        }
-        if (mc.ncs > 0) {
-          b.CSpi2AvI = red[RED_PI2CS];
-          b.CSpi2AvSI = b.CSpi2AvI;
-          b.CSgrad2AvI = red[RED_GRAD2CS];
-        }
-        break;
-      case OP_KERNEL_ONLY:
-        st->K = sf_kernel(b, mc);
-        break;
-      case OP_PV_SF_FIRST:  // positionverlet.h:196-209; the first drift of the stage uses aI before it
-        a_drift = b.aI;
-        b.aIM = b.aI;
-        b.aI += dt / 2.0 * b.aDotI * w;
-        b.aSI = b.aI;
-        break;
-      case OP_PV_MID: {  // positionverlet.h:73-94
-        // storeFieldsAveragesHalf (positionverlet.h:258-266): the half-step field averages feed getSI
-        const double g2SI = red[RED_GRAD2S], cg2SI = red[RED_GRAD2CS], b2SI = red[RED_B2U1];
-        b.potAvSI = red[RED_POT];
-        // storeMomentaAverages (positionverlet.h:238-256)
-        const double pIM = b.pi2AvI, cIM = b.CSpi2AvI, uIM = b.U1pi2AvI;
-        if (mc.ns > 0) b.pi2AvI = red[RED_PI2S];
-        if (mc.ncs > 0) b.CSpi2AvI = red[RED_PI2CS];
-        if (mc.nu1 > 0) b.U1pi2AvI = red[RED_PI2U1];
-        b.pi2AvSI = 0.5 * (b.pi2AvI + pIM);
-        b.CSpi2AvSI = 0.5 * (b.CSpi2AvI + cIM);
-        b.U1pi2AvSI = 0.5 * (b.U1pi2AvI + uIM);
-        // kickScaleFactor with ScaleFactorKernels::getSI (positionverlet.h:151-154)
-        st->K = sf_kernel_of(b.aI, b.pi2AvSI, g2SI, b.CSpi2AvSI, cg2SI, b.U1pi2AvSI, b2SI, b.potAvSI, mc);
-        b.aDotI += dt * st->K * w;
-        // driftScaleFactorSecondHalf (positionverlet.h:212-223); the second drift uses the new aI
-        b.aI += dt / 2.0 * b.aDotI * w;
-        b.aSI = (b.aIM + b.aI) / 2.0;
-        a_drift = b.aI;
-        break;
+  switch (op) {
+    case OP_STORE_FIELDS:  // leapfrog.h:269-277
+      if (mc.ns > 0) b.grad2AvI = red[RED_GRAD2S];
+      if (mc.ncs > 0) b.CSgrad2AvI = red[RED_GRAD2CS];
+      if (mc.nu1 > 0) b.U1Mag2AvI = red[RED_B2U1];
+      b.potAvI = red[RED_POT];
+      break;
+    case OP_LF_MOMENTA:  // leapfrog.h:239-267 then 124-129 and 168-184
+      if (mc.ns > 0) {
+        b.pi2AvSIM = b.pi2AvSI;
+        b.pi2AvSI = red[RED_PI2S];
+        b.pi2AvI = 0.5 * (b.pi2AvSIM + b.pi2AvSI);
       }
-      case OP_PV_DRIFT_AI:
-        a_drift = b.aI;
-        break;
-      default:
-        break;
+      if (mc.ncs > 0) {
+        b.CSpi2AvSIM = b.CSpi2AvSI;
+        b.CSpi2AvSI = red[RED_PI2CS];
+        b.CSpi2AvI = 0.5 * (b.CSpi2AvSIM + b.CSpi2AvSI);
+      }
+      if (mc.nu1 > 0) {
+        b.U1pi2AvSIM = b.U1pi2AvSI;
+        b.U1pi2AvSI = red[RED_PI2U1];
+        b.U1pi2AvI = 0.5 * (b.U1pi2AvSIM + b.U1pi2AvSI);
+      }
+      st->K = sf_kernel<INT>(b, mc);
+      b.aDotSIM = b.aDotSI;
+      b.aDotSI += dt * st->K;
+      b.aDotI = (b.aDotSIM + b.aDotSI) / 2.0;
+      b.aIM = b.aI;
+      b.aI += dt * b.aDotSI;
+      b.aSI = (b.aIM + b.aI) / 2.0;
+      break;
+    case OP_LF_SYNC:  // leapfrog.h:105-112
+      if (mc.ns > 0) b.pi2AvI = red[RED_PI2S];
+      if (mc.ncs > 0) b.CSpi2AvI = red[RED_PI2CS];
+      if (mc.nu1 > 0) b.U1pi2AvI = red[RED_PI2U1];
+      st->K = sf_kernel<INT>(b, mc);
+      b.aDotI = b.aDotSI + dt / 2.0 * st->K;
+      break;
+    case OP_LF_INIT:  // leapfrog.h:35
+      st->K = sf_kernel<INT>(b, mc);
+      b.aDotSI = b.aDotI - dt / 2.0 * st->K;
+      break;
+    case OP_VV_SF_HALF:  // velocityverlet.h:165-168
+      st->K = sf_kernel<INT>(b, mc);
+      b.aDotSI = b.aDotI + (dt / 2) * st->K * w;
+      break;
+    case OP_VV_MOMENTA:  // velocityverlet.h:249-256
+      if (mc.ns > 0) b.pi2AvI = red[RED_PI2S];
+      if (mc.ncs > 0) b.CSpi2AvI = red[RED_PI2CS];
+      if (mc.nu1 > 0) b.U1pi2AvI = red[RED_PI2U1];
+      break;
+    case OP_VV_MOMENTA_KICK2:  // velocityverlet.h:249-256, scalar singlets only
+      b.pi2AvI = red[RED_PI2S_KICK2];
+      break;
+    case OP_VV_DRIFT_SF:  // velocityverlet.h:239-242
+      b.aIM = b.aI;
+      b.aI += dt * b.aDotSI * w;
+      b.aSI = (b.aIM + b.aI) / 2.0;
+      break;
+    case OP_VV_SF_ONE:  // velocityverlet.h:171-174
+      st->K = sf_kernel<INT>(b, mc);
+      b.aDotI = b.aDotSI + (dt / 2) * st->K * w;
+      break;
+    case OP_SET_ALL:  // averages.h:86-116
+      b.potAvI = red[RED_POT];
+      b.potAvSI = b.potAvI;
+      if (mc.ns > 0) {
+        b.pi2AvI = red[RED_PI2S];
+        b.pi2AvSI = b.pi2AvI;
+        b.grad2AvI = red[RED_GRAD2S];
+      }
+      if (mc.nu1 > 0) {
+        b.U1pi2AvI = red[RED_PI2U1];
+        b.U1pi2AvSI = b.U1pi2AvI;
+        b.U1Mag2AvI = red[RED_B2U1];
+      }
+      if (mc.ncs > 0) {
+        b.CSpi2AvI = red[RED_PI2CS];
+        b.CSpi2AvSI = b.CSpi2AvI;
+        b.CSgrad2AvI = red[RED_GRAD2CS];
+      }
+      break;
+    case OP_KERNEL_ONLY:
+      st->K = sf_kernel<INT>(b, mc);
+      break;
+    case OP_PV_SF_FIRST:  // positionverlet.h:196-209; the first drift of the stage uses aI before it
+      a_drift = b.aI;
+      b.aIM = b.aI;
+      b.aI += dt / 2.0 * b.aDotI * w;
+      b.aSI = b.aI;
+      break;
+    case OP_PV_MID: {  // positionverlet.h:73-94
+      // storeFieldsAveragesHalf (positionverlet.h:258-266): the half-step field averages feed getSI
+      const double g2SI = red[RED_GRAD2S], cg2SI = red[RED_GRAD2CS], b2SI = red[RED_B2U1];
+      b.potAvSI = red[RED_POT];
+      // storeMomentaAverages (positionverlet.h:238-256)
+      const double pIM = b.pi2AvI, cIM = b.CSpi2AvI, uIM = b.U1pi2AvI;
+      if (mc.ns > 0) b.pi2AvI = red[RED_PI2S];
+      if (mc.ncs > 0) b.CSpi2AvI = red[RED_PI2CS];
+      if (mc.nu1 > 0) b.U1pi2AvI = red[RED_PI2U1];
+      b.pi2AvSI = 0.5 * (b.pi2AvI + pIM);
+      b.CSpi2AvSI = 0.5 * (b.CSpi2AvI + cIM);
+      b.U1pi2AvSI = 0.5 * (b.U1pi2AvI + uIM);
+      // kickScaleFactor with ScaleFactorKernels::getSI (positionverlet.h:151-154)
+      st->K = sf_kernel_of<INT>(b.aI, b.pi2AvSI, g2SI, b.CSpi2AvSI, cg2SI, b.U1pi2AvSI, b2SI, b.potAvSI, mc);
+      b.aDotI += dt * st->K * w;
+      // driftScaleFactorSecondHalf (positionverlet.h:212-223); the second drift uses the new aI
+      b.aI += dt / 2.0 * b.aDotI * w;
+      b.aSI = (b.aIM + b.aI) / 2.0;
+      a_drift = b.aI;
+      break;
     }
-    if (o == 0 && ops.snap) *ops.snap = b;
+    case OP_PV_DRIFT_AI:
+      a_drift = b.aI;
+      break;
+    default:
+      break;
   }
-  // a^(1+alpha) and a^(3+alpha) = a^(1+alpha) a^2, a^(alpha-1); the drift factors likewise share one power
-  const double aK = rpow(b.aI, 1 + mc.alpha);
+}
+
+// The kick and drift coefficients the next pass reads: a^(1+alpha) and a^(3+alpha) = a^(1+alpha) a^2,
+// a^(alpha-1); the drift factors likewise share one power.
+template <bool INT>
+__device__ __forceinline__ void refresh_coefficients(DevState *st, const ModelConsts &mc, double a_drift)
+{
+  const clmi_background &b = st->bg;
+  const double aK = bg_pow<INT>(b.aI, 1 + mc.alpha);
   st->aK = aK;
   st->aV = aK * (b.aI * b.aI);
-  st->aG = rpow(b.aI, mc.alpha - 1);
+  st->aG = bg_pow<INT>(b.aI, mc.alpha - 1);
   st->aJ = aK;
   const double ad = a_drift > 0.0 ? a_drift : b.aSI;
-  const double fu = rpow(ad, mc.alpha - 1);
+  const double fu = bg_pow<INT>(ad, mc.alpha - 1);
   st->fdrift_u = fu;
   st->fdrift_s = fu / (ad * ad);
+}
+
+// Executed by one thread: the operations in order, then the coefficients.
+__device__ inline void apply_update(DevState *st, const double *red, const ModelConsts &mc, const UpdateOps &ops)
+{
+  double a_drift = -1.0;
+  for (int o = 0; o < ops.n; ++o) {
+    apply_op<false>(st, red, mc, ops.op[o], ops.w[o], a_drift);
+    if (o == 0 && ops.snap) *ops.snap = st->bg;
+  }
+  refresh_coefficients<false>(st, mc, a_drift);
 }
 
 }  // namespace clmi

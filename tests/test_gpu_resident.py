@@ -1,0 +1,100 @@
+"""The resident evolver (one launch for many passes of a lattice of side <= 128, scalar_resident.hpp) against
+the pass-by-pass evolvers, which a context with pass timing on runs: the same operations in the same order, so
+fields, momenta, background and constraint agree to the bit."""
+import threading
+
+import numpy as np
+import pytest
+
+from cosmolattice_amd.clmi import (CLMI_F32_BULK, CLMI_F64, FLD_S, PI_S, PV_WEIGHTS, VV_WEIGHTS, Lattice,
+                                   lphi4)
+
+pytestmark = pytest.mark.gpu
+
+
+def model(kind):
+    base = lphi4(100.0, n_fields=1 if kind == "1f" else 2, phi0_gev=5.6964e18, lam=1.0, pi0_program=-0.5)
+    if kind == "terms":  # outside the compile-time potential
+        base.terms = [(0.25, [4, 0]), (50.0, [2, 2]), (0.1, [0, 4]), (0.3, [2, 0])]
+    return base
+
+
+def start(spec, N, prec, expansion, seed=5):
+    rng = np.random.default_rng(seed)
+    lat = Lattice(spec, N, 0.4909, 0.005, prec, expansion=expansion)
+    for k in (FLD_S, PI_S):
+        for f in range(spec.n_scalars):
+            lat.upload(k, f, 0, 0.3 * rng.standard_normal((N, N, N)) + (1.0 if k == FLD_S and f == 0 else 0.0))
+    lat.set_background(aI=1.0, aSI=1.0, aIM=1.0, aDotI=0.7)
+    lat.set_all_averages()
+    return lat
+
+
+def evolve(lat, scheme):
+    """Calls of uneven length around the fewest passes the resident evolver takes, then the whole state."""
+    for n in (6, 1, 5, 9):
+        if scheme == "LF":
+            if n == 6:
+                lat.lf_init()
+            lat.lf_evolve(n)
+            if n == 5:
+                lat.lf_sync()
+        elif scheme.startswith("VV"):
+            lat.vv_evolve(VV_WEIGHTS[scheme], n)
+        else:
+            lat.pv_evolve(PV_WEIGHTS[scheme], n)
+    if scheme == "LF":
+        lat.lf_sync()
+    fields = [lat.download(k, f, 0) for k in (FLD_S, PI_S) for f in range(lat.spec.n_scalars)]
+    return fields, lat.background(), lat.hubble_constraint()
+
+
+@pytest.mark.parametrize("N", [64, 128])
+@pytest.mark.parametrize("prec", [CLMI_F64, CLMI_F32_BULK])
+@pytest.mark.parametrize("kind,scheme,expansion", [("2f", "LF", True), ("1f", "LF", True), ("terms", "LF", False),
+                                                   ("2f", "VV4", True), ("1f", "VV2", True), ("2f", "PV4", True),
+                                                   ("1f", "PV2", False)])
+def test_resident_bit_identical_to_passes(gpu, N, prec, kind, scheme, expansion):
+    print(f"case resident N={N} prec={prec} {kind} {scheme} expansion={expansion}", flush=True)
+    spec = model(kind)
+    res = []
+    for timed in (False, True):
+        lat = start(spec, N, prec, expansion)
+        assert "k_scalar_resident" in lat.plan()
+        if timed:
+            lat.profile_enable(True, every=1 << 30)
+        res.append(evolve(lat, scheme))
+        lat.close()
+    (fa, ba, ca), (fb, bb, cb) = res
+    for a, b in zip(fa, fb):
+        assert np.array_equal(a, b)
+    assert ba == bb and ca == cb
+    if expansion:
+        assert ba["aI"] > 1.0
+
+
+def test_resident_two_threads(gpu):
+    """Two contexts driven by two host threads at once: each ends where it ends alone."""
+    print("case resident two threads", flush=True)
+    spec = model("2f")
+
+    def run(seed, out):
+        lat = start(spec, 128, CLMI_F32_BULK, True, seed)
+        lat.lf_init()
+        for _ in range(10):
+            lat.lf_evolve(20)
+        lat.lf_sync()
+        out[seed] = [lat.download(k, f, 0) for k in (FLD_S, PI_S) for f in range(2)]
+        lat.close()
+
+    alone, together = {}, {}
+    for seed in (1, 2):
+        run(seed, alone)
+    threads = [threading.Thread(target=run, args=(seed, together)) for seed in (1, 2)]
+    for t in threads:
+        t.start()
+    for t in threads:
+        t.join()
+    for seed in (1, 2):
+        for a, b in zip(alone[seed], together[seed]):
+            assert np.array_equal(a, b)
