@@ -29,6 +29,11 @@ HIP_SOURCES = [
     "scalar_rows_f64.hip",
     "scalar_rows_f64_1f.hip",
     "scalar_rows_batch.hip",
+    "scalar_flat.hip",
+    "scalar_flat_f32.hip",
+    "scalar_flat_f32_1f.hip",
+    "scalar_flat_f64.hip",
+    "scalar_flat_f64_1f.hip",
     "scalar_resident.hip",
     "scalar_resident_lf_f64.hip",
     "scalar_resident_lf_f32.hip",

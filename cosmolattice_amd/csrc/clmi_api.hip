@@ -54,6 +54,8 @@ struct clmi_ctx {
   TiledPlan tplan;
   bool rowk = false;   // scalar passes use the full-row kernel with plan rplan
   RowsPlan rplan;
+  bool flat = false;   // scalar passes use the plane-chunk kernel with plan fplan
+  FlatPlan fplan;
   bool gtiled = false; // charged scalar + U(1) passes use the tiled kernel (gTY-row tiles, x-chunk gXC)
   int gTY = 4;
   int gXC = 0;
@@ -277,8 +279,8 @@ int run_pass(clmi_ctx *c, bool drift, bool kick, bool red, double cdt_s, double 
              double ckick2_s = 0.0)
 {
   const bool kick2 = ckick2_s != 0.0;
-  if (kick2 && !(drift && kick && (c->rowk || c->tiled) && c->cfg.n_cscalars == 0))
-    return fail(c, CLMI_E_INVALID, "double kick outside a scalar-singlet full-row or tiled drift + kick pass");
+  if (kick2 && !(drift && kick && (c->rowk || c->tiled || c->flat) && c->cfg.n_cscalars == 0))
+    return fail(c, CLMI_E_INVALID, "double kick outside a scalar-singlet full-row, tiled or plane-chunk drift + kick pass");
   const bool timed = c->prof && drift && kick && (c->prof_count++ % c->prof_every == 0);
   if (timed) CHK(prof_event(c));
   int r = 0;
@@ -287,7 +289,7 @@ int run_pass(clmi_ctx *c, bool drift, bool kick, bool red, double cdt_s, double 
     const int pi = c->cur_pS, po = (drift && kick) ? 1 - c->cur_pS : c->cur_pS;
     ScalarPassArgs a = scalar_args(c, fi, fo, pi, po, cdt_s, ckick_s, r);
     a.ckick2 = ckick2_s;
-    const int nrows = c->rowk ? c->rplan.rows : c->tiled ? c->tplan.rows : c->blocks_s;
+    const int nrows = c->rowk ? c->rplan.rows : c->tiled ? c->tplan.rows : c->flat ? c->fplan.rows : c->blocks_s;
     if (red && (size_t)r + nrows > c->partial_rows)
       return fail(c, CLMI_E_INVALID, "partial-sum buffer too small for the scalar pass");
     if (c->rowk) {
@@ -296,6 +298,9 @@ int run_pass(clmi_ctx *c, bool drift, bool kick, bool red, double cdt_s, double 
     } else if (c->tiled) {
       HIPCHK(c, launch_scalar_tiled(c->cfg.n_scalars, c->f32, drift, kick, red, a, c->tplan, c->stream, kick2));
       if (red) r += c->tplan.rows;
+    } else if (c->flat) {
+      HIPCHK(c, launch_scalar_flat(c->cfg.n_scalars, c->f32, drift, kick, red, a, c->fplan, c->stream, kick2));
+      if (red) r += c->fplan.rows;
     } else {
       HIPCHK(c, launch_scalar_pass(c->cfg.n_scalars, c->f32, drift, kick, red, a, c->blocks_s, c->stream));
       if (red) r += c->blocks_s;
@@ -358,11 +363,11 @@ int pass_update(clmi_ctx *c, bool drift, bool kick, bool red, double cdt_s, doub
   return CLMI_OK;
 }
 
-// Whether velocity-Verlet stages may share a double-kick pass: scalar singlets only, on the full-row or
-// the tiled pass.
+// Whether velocity-Verlet stages may share a double-kick pass: scalar singlets only, on the full-row, the
+// tiled or the plane-chunk pass.
 bool double_kick_ok(const clmi_ctx *c)
 {
-  return (c->rowk || c->tiled) && c->cfg.n_scalars > 0 && c->cfg.n_cscalars == 0 && !(c->cfg.flags & CLMI_FLAG_NO_DOUBLE_KICK);
+  return (c->rowk || c->tiled || c->flat) && c->cfg.n_scalars > 0 && c->cfg.n_cscalars == 0 && !(c->cfg.flags & CLMI_FLAG_NO_DOUBLE_KICK);
 }
 
 // Fewest passes that the resident evolver takes: a cooperative launch with its load and store of the state costs
@@ -608,6 +613,7 @@ int clmi_create(const clmi_config *cfg, clmi_ctx **out)
           c->tplan = p;
           break;
         }
+    if (!c->rowk && !c->tiled && scalar_flat_plan(g.N, g.n_scalars, ncu, &c->fplan)) c->flat = true;
     int gxc = 0, gblocks = 0, grows_t = 0;
     const int gty = (g.flags & CLMI_FLAG_GAUGE_TY8) ? 8 : 4;
     if (g.n_cscalars > 0 && gauge_tiled_plan(g.N, gty, ncu, &gxc, &gblocks, &grows_t)) {
@@ -620,7 +626,7 @@ int clmi_create(const clmi_config *cfg, clmi_ctx **out)
   }
   // The resident evolver: integer alpha (its background update has no general power), a CU for every tile (the
   // launch itself checks that they fit).
-  if (!(g.flags & (CLMI_FLAG_NO_TILED | CLMI_FLAG_NO_DOUBLE_KICK)) && g.n_cscalars == 0 && g.N % 64 == 0 &&
+  if (!(g.flags & (CLMI_FLAG_NO_TILED | CLMI_FLAG_NO_DOUBLE_KICK)) && g.n_cscalars == 0 &&
       g.alpha == std::rint(g.alpha) && std::fabs(g.alpha) <= 15.0 && resident_plan(g.N, g.n_scalars, &c->resp)) {
     int cus = 0, coop = 0;
     c->resident = hipDeviceGetAttribute(&cus, hipDeviceAttributeMultiprocessorCount, c->device) == hipSuccess &&
@@ -632,6 +638,7 @@ int clmi_create(const clmi_config *cfg, clmi_ctx **out)
   const size_t srows = g.n_scalars == 0 ? 0
                        : c->rowk        ? (size_t)c->rplan.rows
                        : c->tiled       ? (size_t)c->tplan.rows
+                       : c->flat        ? (size_t)c->fplan.rows
                                         : (size_t)c->blocks_s;
   const size_t grows = g.n_cscalars > 0 ? (size_t)c->rows_g : 0;
   const size_t rows = std::max(2 * (size_t)kMaxPassBlocks, srows + grows) + 16;
@@ -2269,6 +2276,9 @@ int clmi_plan_report(const clmi_ctx *c, char *report, size_t report_len)
       rep += "k_scalar_tiled XC=" + std::to_string(c->tplan.XC) + " G=" + std::to_string(c->tplan.G) +
              " NT=" + std::to_string((int)c->tplan.NT) + " PK=" + std::to_string(poly_kind(c->spoly, c->cfg.n_scalars)) +
              "\n";
+    else if (c->flat)
+      rep += "k_scalar_flat VZ=" + std::to_string(c->fplan.VZ) + " XC=" + std::to_string(c->fplan.XC) +
+             " G=" + std::to_string(c->fplan.G) + " PK=" + std::to_string(poly_kind(c->spoly, c->cfg.n_scalars)) + "\n";
     else
       rep += "k_scalar_pass\n";
     if (c->resident)

@@ -257,7 +257,7 @@ struct ResidentArgs {
 // Tiles of the resident evolver for an N^3 lattice: chunks of kResThreads * VZ sites of a plane by P planes.
 struct ResidentPlan {
   int VZ = 0, P = 0, groups = 0, chunks = 0;
-  bool ragged = false;  // tiles that are not full
+  bool ragged = false;  // some tiles may not be full
 };
 bool resident_plan(int N, int nf, ResidentPlan *p);
 // hipErrorCooperativeLaunchTooLarge where the device does not hold all tiles at once.
@@ -386,6 +386,16 @@ hipError_t launch_scalar_rows(int nf, bool f32, bool drift, bool kick, bool red,
                               const RowsPlan &p, hipStream_t s, bool kick2 = false);
 hipError_t launch_scalar_tiled(int nf, bool f32, bool drift, bool kick, bool red, const ScalarPassArgs &a,
                                const TiledPlan &p, hipStream_t s, bool kick2 = false);
+constexpr int kFlatThreads = 512;
+struct FlatPlan {  // plane-chunk pass (scalar_flat.hpp)
+  int VZ = 0, XC = 0, G = 0;
+  int chunks = 0;   // workgroups per plane
+  bool NT = false;  // non-temporal stores
+  int blocks = 0, rows = 0;
+};
+bool scalar_flat_plan(int N, int nf, int ncu, FlatPlan *p);
+hipError_t launch_scalar_flat(int nf, bool f32, bool drift, bool kick, bool red, const ScalarPassArgs &a,
+                              const FlatPlan &p, hipStream_t s, bool kick2 = false);
 hipError_t launch_copy(const void *src, void *dst, size_t bytes, hipStream_t s);
 // Copies of up to kCopySetMax device arrays in one launch (sizes in 16-byte units).
 constexpr int kCopySetMax = 12;

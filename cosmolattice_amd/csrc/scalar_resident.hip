@@ -23,21 +23,23 @@ const void *kernel_of(int scheme, int nf, bool f32, int pk, const ResidentPlan &
 }
 }  // namespace
 
-// One site per lane up to 64^3, two above (64 and 128 as the full-row pass has them).  Four planes per tile
-// where that gives at most 256 tiles -- one per CU, and half the sites per wave of eight-plane tiles --
-// else eight; 64^3 and 128^3 take eight, the full-row pass's group, so that their sums are the same.
+// One site per lane up to 64^3, two above (64 and 128 as the full-row pass has them).  64^3 and 128^3 take
+// eight planes per tile, the full-row pass's group, so that their sums are the same.  Others take four where
+// that gives at most 256 tiles, one per CU and half the sites per wave of eight (100^3 FP64: 13.3 us a step), else
+// eight; up to 40^3 two, which the plane-chunk pass needs (its tile is the same): at 32^3, two fields FP64, a pass
+// and its update take 11.1 us with two planes and 12.8 with four, the resident step 4.8 and 5.2.
 bool resident_plan(int N, int nf, ResidentPlan *p)
 {
   if (nf < 1 || nf > 2 || N < 24 || N > 128 || (N & 1)) return false;
   p->VZ = N <= 64 ? 1 : 2;
   const int C = kResThreads * p->VZ;
   p->chunks = (N * N + C - 1) / C;
-  for (int P : {4, 8}) {
+  for (int P : {N <= 40 ? 2 : 4, 8}) {
     p->P = P;
     p->groups = (N + P - 1) / P;
     if (N % 64 != 0 && p->groups * p->chunks <= 256) break;
   }
-  p->ragged = N % p->P != 0 || (N * N) % C != 0;
+  p->ragged = N % 64 != 0;  // (every tile of 64^3 and 128^3 is full)
   return p->groups * p->chunks <= 256;
 }
 

@@ -664,6 +664,7 @@ template <int NF, bool F32, int SCH, int PK>
 const void *resident_shape(const ResidentPlan &p)
 {
   switch (p.VZ * 100 + p.P * 10 + (p.ragged ? 1 : 0)) {
+    case 121: return (const void *)k_scalar_resident<NF, F32, 1, 2, true, PK, SCH>;
     case 141: return (const void *)k_scalar_resident<NF, F32, 1, 4, true, PK, SCH>;
     case 180: return (const void *)k_scalar_resident<NF, F32, 1, 8, false, PK, SCH>;
     case 241: return (const void *)k_scalar_resident<NF, F32, 2, 4, true, PK, SCH>;

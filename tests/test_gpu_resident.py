@@ -1,13 +1,14 @@
-"""The resident evolver (one launch for many passes of a lattice of side <= 128, scalar_resident.hpp) against
-the pass-by-pass evolvers, which a context with pass timing on runs: the same operations in the same order, so
-fields, momenta, background and constraint agree to the bit."""
+"""The resident evolver (one launch for many passes of a lattice of side <= 128, scalar_resident.hpp) and the
+plane-chunk pass of ragged sides (scalar_flat.hpp).  The resident evolver is compared with the pass-by-pass
+evolvers, which a context with pass timing on runs: the same operations in the same order, so fields, momenta,
+background and constraint agree to the bit."""
 import threading
 
 import numpy as np
 import pytest
 
-from cosmolattice_amd.clmi import (CLMI_F32_BULK, CLMI_F64, FLD_S, PI_S, PV_WEIGHTS, VV_WEIGHTS, Lattice,
-                                   lphi4)
+from cosmolattice_amd.clmi import (CLMI_F32_BULK, CLMI_F64, CLMI_FLAG_NO_TILED, FLD_S, PI_S, PV_WEIGHTS, VV_WEIGHTS,
+                                   Lattice, lphi4)
 
 pytestmark = pytest.mark.gpu
 
@@ -49,7 +50,7 @@ def evolve(lat, scheme):
     return fields, lat.background(), lat.hubble_constraint()
 
 
-@pytest.mark.parametrize("N", [64, 128])
+@pytest.mark.parametrize("N", [32, 64, 100, 120, 128])
 @pytest.mark.parametrize("prec", [CLMI_F64, CLMI_F32_BULK])
 @pytest.mark.parametrize("kind,scheme,expansion", [("2f", "LF", True), ("1f", "LF", True), ("terms", "LF", False),
                                                    ("2f", "VV4", True), ("1f", "VV2", True), ("2f", "PV4", True),
@@ -71,6 +72,48 @@ def test_resident_bit_identical_to_passes(gpu, N, prec, kind, scheme, expansion)
     assert ba == bb and ca == cb
     if expansion:
         assert ba["aI"] > 1.0
+
+
+# chunk and group edges: one chunk per plane (24), chunks ending inside a row, full chunks (32, 96), the widest one-site
+# and two-site lanes (62, 126), eight-plane tiles with a short last group (126), and sizes past the resident evolver
+@pytest.mark.parametrize("N", [24, 32, 42, 62, 66, 96, 100, 126, 130, 250, 300])
+@pytest.mark.parametrize("prec", [CLMI_F64, CLMI_F32_BULK])
+@pytest.mark.parametrize("kind,scheme", [("2f", "LF"), ("1f", "VV2"), ("terms", "PV2")])
+def test_ragged_sides_bit_identical_to_one_site_per_thread(gpu, N, prec, kind, scheme):
+    """The plane-chunk pass, pass by pass and (N <= 128) in the resident evolver, on a static background: fields
+    and momenta equal the one-site-per-thread pass's to the bit; its sums differ in order only."""
+    print(f"case ragged N={N} prec={prec} {kind} {scheme}", flush=True)
+    spec = model(kind)
+    rng = np.random.default_rng(N)
+    ics = {(k, f): 0.3 * rng.standard_normal((N, N, N)) + (1.0 if (k, f) == (FLD_S, 0) else 0.0)
+           for k in (FLD_S, PI_S) for f in range(spec.n_scalars)}
+    res = []
+    for how in ("one site", "passes", "default"):
+        lat = Lattice(spec, N, 0.4909, 0.005, prec, expansion=False, flags=CLMI_FLAG_NO_TILED if how == "one site" else 0)
+        plan = lat.plan()
+        assert plan.split()[0] == ("k_scalar_pass" if how == "one site" else "k_scalar_flat")
+        assert ("k_scalar_resident" in plan) == (how != "one site" and N <= 128)
+        for (k, f), a in ics.items():
+            lat.upload(k, f, 0, a)
+        lat.set_background(aI=1.1, aSI=1.05, aIM=1.0)
+        if how == "passes":
+            lat.profile_enable(True, every=1 << 30)
+        if scheme == "LF":
+            lat.lf_init()
+            lat.lf_evolve(6)
+            lat.lf_sync()
+        elif scheme == "VV2":
+            lat.vv_evolve([1.0], 6)
+        else:
+            lat.pv_evolve([1.0], 4)
+        res.append(([lat.download(k, f, 0) for k, f in ics], lat.averages()))
+        lat.close()
+    for fields, sums in res[1:]:
+        for a, b in zip(res[0][0], fields):
+            assert np.array_equal(a, b)
+        for k in ("pi2S", "grad2S", "pot"):
+            assert sums[k] == pytest.approx(res[0][1][k], rel=1e-13)
+    assert res[1][1] == res[2][1]
 
 
 def test_resident_two_threads(gpu):
