@@ -613,7 +613,7 @@ int clmi_create(const clmi_config *cfg, clmi_ctx **out)
           c->tplan = p;
           break;
         }
-    if (!c->rowk && !c->tiled && scalar_flat_plan(g.N, g.n_scalars, ncu, &c->fplan)) c->flat = true;
+    if (!c->rowk && !c->tiled && scalar_flat_plan(g.N, g.n_scalars, &c->fplan)) c->flat = true;
     int gxc = 0, gblocks = 0, grows_t = 0;
     const int gty = (g.flags & CLMI_FLAG_GAUGE_TY8) ? 8 : 4;
     if (g.n_cscalars > 0 && gauge_tiled_plan(g.N, gty, ncu, &gxc, &gblocks, &grows_t)) {

@@ -389,11 +389,10 @@ hipError_t launch_scalar_tiled(int nf, bool f32, bool drift, bool kick, bool red
 constexpr int kFlatThreads = 512;
 struct FlatPlan {  // plane-chunk pass (scalar_flat.hpp)
   int VZ = 0, XC = 0, G = 0;
-  int chunks = 0;   // workgroups per plane
-  bool NT = false;  // non-temporal stores
+  int chunks = 0;  // workgroups per plane
   int blocks = 0, rows = 0;
 };
-bool scalar_flat_plan(int N, int nf, int ncu, FlatPlan *p);
+bool scalar_flat_plan(int N, int nf, FlatPlan *p);
 hipError_t launch_scalar_flat(int nf, bool f32, bool drift, bool kick, bool red, const ScalarPassArgs &a,
                               const FlatPlan &p, hipStream_t s, bool kick2 = false);
 hipError_t launch_copy(const void *src, void *dst, size_t bytes, hipStream_t s);

@@ -12,10 +12,12 @@ hipError_t launch_scalar_flat_f32_nf1(bool drift, bool kick, bool red, const Sca
 hipError_t launch_scalar_flat_f32_nf2(bool drift, bool kick, bool red, const ScalarPassArgs &a, const FlatPlan &p,
                                       hipStream_t s, bool kick2);
 
-// Even N from 24 (below, a lattice has fewer sites than a few workgroups' chunks) to 500 (two LDS rows of two fields in 64 KiB).  One site per
-// lane up to N = 64, two above; the resident evolver's groups up to N = 128.  The x-chunk is the longest of up
-// to 32 planes that gives the device's ncu CUs two workgroups each, else one group.
-bool scalar_flat_plan(int N, int nf, int ncu, FlatPlan *p)
+// Even N from 24 (below, a lattice has fewer sites than a few workgroups' chunks) to 500 (two LDS rows of two fields
+// in 64 KiB).  One site per lane up to N = 64, two above; the resident evolver's groups up to N = 128.  The x-chunk
+// is one group: many short marches balance the CUs and keep the x-halo in L2 (us a step, two fields FP64, x-chunk 8
+// / 16 / 24 / 32: 180^3 92 / 96 / 88 / 99, 200^3 119 / 140 / 138 / 158, 250^3 226 / 229 / 250 / 230; 300^3 from 16:
+// 386 / - / 400).
+bool scalar_flat_plan(int N, int nf, FlatPlan *p)
 {
   if (nf < 1 || nf > 2 || (N & 1) || N < 24 || N > 500) return false;
   ResidentPlan r;
@@ -24,12 +26,6 @@ bool scalar_flat_plan(int N, int nf, int ncu, FlatPlan *p)
   const int C = kFlatThreads * p->VZ;
   p->chunks = (N * N + C - 1) / C;
   p->XC = p->G;
-  for (int xc = 32; xc > p->G; xc /= 2)
-    if (xc % p->G == 0 && p->chunks * ((N + xc - 1) / xc) >= 2 * ncu) {
-      p->XC = xc;
-      break;
-    }
-  p->NT = N > 128;  // smaller lattices stay in the memory-side cache from one pass to the next
   p->blocks = p->chunks * ((N + p->XC - 1) / p->XC);
   p->rows = p->chunks * ((N + p->G - 1) / p->G);
   return true;

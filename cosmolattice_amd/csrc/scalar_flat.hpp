@@ -12,15 +12,13 @@
 // from L2: the neighbouring chunk runs on the same XCD) and two planes per x-chunk.
 //
 // Measured (MI355X, leapfrog step, two fields; against one site per thread): 100^3 FP64 33.4 -> 21.5 us, 200^3 FP64
-// 230 -> 140 us (3.7 TB/s of the arrays' bytes), 250^3 FP32-bulk 375 -> 193 us, 300^3 FP64 814 -> 399 us (4.3),
-// 500^3 FP64 3906 -> 1744 us (4.6).  What bounds it is the memory path: halo rows that miss L2, and above 256^3
+// 230 -> 119 us (4.3 TB/s of the arrays' bytes), 250^3 FP32-bulk 375 -> 190 us, 300^3 FP64 814 -> 386 us (4.5),
+// 500^3 FP64 3906 -> 1744 us (4.6).  Non-temporal stores made no difference.  What bounds it is the memory path: halo rows that miss L2, and above 256^3
 // the halo's share of the chunk.
 //
 // Volume sums are written per (group of G planes, chunk), independent of XC; for N <= 128 these are the tiles
 // of the resident evolver, so its sums are the same.
 #pragma once
-
-#include <type_traits>
 
 #include "scalar_site.hpp"
 
@@ -30,7 +28,7 @@ namespace {
 // NH: halo pairs per thread (N * NF pairs in all).
 template <int NF, bool F32, int VZ, int NH, bool DRIFT, bool KICK, bool RED, int PK, bool KICK2 = false>
 __global__ __launch_bounds__(kFlatThreads) void k_scalar_flat(const ScalarPassArgs a, const int XC, const int G,
-                                                              const int chunks, const int nt)
+                                                              const int chunks)
 {
   static_assert(!KICK2 || (DRIFT && KICK), "a double kick follows a drift");
   using T = Tr<F32>;
@@ -157,14 +155,13 @@ __global__ __launch_bounds__(kFlatThreads) void k_scalar_flat(const ScalarPassAr
 #pragma unroll
       for (int f = 0; f < NF; ++f) pout[f][k] = pk[f];
     }
-    auto store = [&](auto ntc) {
-      constexpr bool NTS = decltype(ntc)::value;
+    if (act) {
 #pragma unroll
       for (int f = 0; f < NF; ++f) {
-        if (KICK) vstore<VZ, NTS>((M *)a.pi_out[f], s0, pout[f]);
+        if (KICK) vstore<VZ, false>((M *)a.pi_out[f], s0, pout[f]);
         if (DRIFT) {
           if constexpr (!F32) {
-            vstore<VZ, NTS>((double *)a.phi_out[f], s0, cur[f]);
+            vstore<VZ, false>((double *)a.phi_out[f], s0, cur[f]);
           } else {
             float h[VZ], l[VZ];
 #pragma unroll
@@ -172,15 +169,11 @@ __global__ __launch_bounds__(kFlatThreads) void k_scalar_flat(const ScalarPassAr
               h[k] = cur[f][k].x;
               l[k] = cur[f][k].y;
             }
-            vstore<VZ, NTS>((float *)a.phi_out[f], s0, h);
-            vstore<VZ, NTS>(a.philo_out[f], s0, l);
+            vstore<VZ, false>((float *)a.phi_out[f], s0, h);
+            vstore<VZ, false>(a.philo_out[f], s0, l);
           }
         }
       }
-    };
-    if (act) {
-      if (nt) store(std::true_type{});
-      else store(std::false_type{});
     }
     if (RED) {
       acc[0] += p2;
@@ -218,8 +211,7 @@ hipError_t dispatch_flat(bool drift, bool kick, bool red, const ScalarPassArgs &
 {
   const size_t lds = 2 * (size_t)NF * (kFlatThreads * VZ + 2 * a.N) * 8;
   const dim3 grid(p.blocks), blk(kFlatThreads);
-  const int nt = p.NT ? 1 : 0;
-#define CLMI_SF(...) hipLaunchKernelGGL((k_scalar_flat<NF, F32, VZ, NH, __VA_ARGS__>), grid, blk, lds, s, a, p.XC, p.G, p.chunks, nt)
+#define CLMI_SF(...) hipLaunchKernelGGL((k_scalar_flat<NF, F32, VZ, NH, __VA_ARGS__>), grid, blk, lds, s, a, p.XC, p.G, p.chunks)
   if (kick2) {
     if (!drift || !kick) return hipErrorInvalidValue;
     if (red) CLMI_SF(true, true, true, PK, true);
