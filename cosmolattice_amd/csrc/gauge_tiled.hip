@@ -1,4 +1,4 @@
-// Charged scalar + U(1) lattice pass, x-marching with LDS plane tiles (N a multiple of 64).
+// Charged scalar + U(1) lattice pass, x-marching with LDS plane tiles (gauge_ragged and multiples of 64).
 //
 // A workgroup of TY wavefronts (TY = 4 or 8) owns a tile of TY y-rows x 64 z-sites (one site per
 // lane) and marches along x over XC planes.  The drifted values of all five field components (phi_0, phi_1, A_x, A_y,
@@ -8,7 +8,10 @@
 // field value is loaded from memory and drifted once per tile instead of once per use.  The raw
 // values of plane x+2 are loaded while plane x is computed; the momenta of a thread's own site stay
 // in registers from that load until the kick uses them.  The per-site arithmetic is
-// gauge_site.hpp's, so fields are bit-identical to the one-site-per-thread pass.  Volume sums are
+// gauge_site.hpp's, so fields are bit-identical to the one-site-per-thread pass.  Where N is no multiple of 64
+// (RAG) a row is cut into equal tiles of at most 64 sites and the last tile of rows and x-chunk may be short
+// (us a step against the one-site pass: 100^3 FP64 73 / 112, 200^3 FP64 445 / 900, 250^3 FP32-bulk 664 / 1464); the
+// idle lanes (14 of 64 at N = 100) cost less than the neighbours' reads of the one-site pass.  Volume sums are
 // written per (group of G planes, tile), so they do not depend on the x-chunk XC: every XC gives the
 // same partial rows in the same order, and the autotuner may pick any of them.
 #include <algorithm>
@@ -19,10 +22,16 @@ namespace clmi {
 namespace {
 
 constexpr int GTZ = 64;  // z sites per tile (one per lane)
+// Whether a side that is no multiple of 64 takes the tiled pass: from 52 (48^3 FP64: 24.5 us a step against 21.8 one
+// site per thread; 56^3: 26 against 32), but not just above 64, where a row is two tiles with half their lanes
+// (66^3 FP32-bulk: 39 against 35 us; 80^3: 39 against 53).
+constexpr bool gauge_ragged(int N) { return N >= 52 && !(N > 64 && N < 76); }
 // planes per partial-sum row: the largest power of two (so that it divides N, a multiple of 64) not
-// above N/8, between 8 and 32 (2048 rows at 256^3 for the background update)
+// above N/8, between 8 and 32 (2048 rows at 256^3 for the background update); for other N four up to 128 and
+// eight above, which leaves the x-chunk, a multiple of it, room to fit the device (see gauge_tiled_plan)
 inline int gauge_rows_g(int N)
 {
+  if (N % GTZ != 0) return N <= 128 ? 4 : 8;
   const int target = std::min(32, N / 8);
   int G = 8;
   while (2 * G <= target) G *= 2;
@@ -78,21 +87,27 @@ template <> struct GRaw<true> {
 
 // Outputs are written with non-temporal stores: nothing in the pass reads them back, and keeping them
 // out of L2 leaves room for the halo rows that neighbouring tiles re-read (256^3: 663 -> 643 us FP64,
-// 474 -> 461 us FP32-bulk).
-template <bool F32> __device__ __forceinline__ void nt_store_v(void *f, float *lo, uint32_t i, typename GVal<F32>::V v)
+// 474 -> 461 us FP32-bulk).  Ragged rows use ordinary stores: their tiles end inside cache lines, whose two parts
+// then meet in L2 (100^3 FP32-bulk 69 -> 60 us a step, 250^3 713 -> 664).
+template <bool NT, class T> __device__ __forceinline__ void store_out(T *p, T v)
+{
+  if constexpr (NT) __builtin_nontemporal_store(v, p);
+  else *p = v;
+}
+template <bool F32, bool NT> __device__ __forceinline__ void store_v(void *f, float *lo, uint32_t i, typename GVal<F32>::V v)
 {
   if constexpr (F32) {
-    __builtin_nontemporal_store(v.h, (float *)f + i);
-    __builtin_nontemporal_store(v.l, lo + i);
+    store_out<NT>((float *)f + i, v.h);
+    store_out<NT>(lo + i, v.l);
   } else {
-    __builtin_nontemporal_store(v, (double *)f + i);
+    store_out<NT>((double *)f + i, v);
   }
 }
 
 // U1: the lattice has a U(1) field, known at compile time (1) or read from the arguments (0).  Fixing it
 // removes the per-site selects and branches on it; that pays for FP32-bulk (256^3 pass 479 -> 462 us)
 // and not for FP64 (670 -> 683 us), so only FP32-bulk lattices with a U(1) field use U1 = 1.
-template <bool F32, bool DRIFT, bool KICK, bool RED, int GTY, int U1 = 0>
+template <bool F32, bool DRIFT, bool KICK, bool RED, int GTY, int U1 = 0, bool RAG = false>
 __global__ __launch_bounds__(64 * GTY) void k_gauge_tiled(const GaugePassArgs a, const int XC, const int RG)
 {
   using G = GVal<F32>;
@@ -103,13 +118,18 @@ __global__ __launch_bounds__(64 * GTY) void k_gauge_tiled(const GaugePassArgs a,
 
   const int N = (int)a.N;
   const uint32_t NN = (uint32_t)N * N;
-  const int nTz = N / GTZ, nTy = N / GTY;
+  const int nTz = RAG ? (N + GTZ - 1) / GTZ : N / GTZ, nTy = RAG ? (N + GTY - 1) / GTY : N / GTY;
   const int nwg = gridDim.x, b = blockIdx.x;
   const int L = (nwg % 8 == 0) ? (b % 8) * (nwg / 8) + b / 8 : b;
   const int tz = L % nTz, ty = (L / nTz) % nTy, cx = L / (nTz * nTy);
-  const int z0 = tz * GTZ, y0 = ty * GTY, x0 = cx * XC;
+  // tile: TW x TH sites, planes x0 .. xe - 1
+  const int tw = RAG ? (N + nTz - 1) / nTz : GTZ;
+  const int z0 = tz * tw, y0 = ty * GTY, x0 = cx * XC;
+  const int TW = RAG ? min(tw, N - z0) : GTZ, TH = RAG ? min(GTY, N - y0) : GTY, xe = RAG ? min(x0 + XC, N) : x0 + XC;
   const int t = threadIdx.x, lane = t & 63, wave = t >> 6;
-  const int y = y0 + wave, z = z0 + lane;
+  // threads outside a short tile load its last site again, and neither write nor count anything
+  const bool act = !RAG || (lane < TW && wave < TH);
+  const int y = y0 + (RAG ? min(wave, TH - 1) : wave), z = z0 + (RAG ? min(lane, TW - 1) : lane);
   GaugeK k = gauge_consts(a, KICK);
   if constexpr (U1 == 1) k.u1 = true;
   const bool u1 = k.u1;
@@ -129,25 +149,25 @@ __global__ __launch_bounds__(64 * GTY) void k_gauge_tiled(const GaugePassArgs a,
     return (uint32_t)wrap(xx) * NN + (uint32_t)wrap(yy) * N + (uint32_t)wrap(zz);
   };
 
-  // halo cell of this thread (2 * 66 + 2 * GTY of 64 * GTY threads): rows y0-1 and y0+GTY with corners,
-  // columns z0-1, z0+64
+  // halo cell of this thread (2 (TW + 2) + 2 TH of 64 GTY threads): rows y0-1 and y0+TH with corners,
+  // columns z0-1, z0+TW
   int hly = -1, hlz = 0, hy = 0, hz = 0;
-  if (t < GTZ + 2) {
+  if (t < TW + 2) {
     hly = 0; hlz = t; hy = y0 - 1; hz = z0 - 1 + t;
-  } else if (t < 2 * (GTZ + 2)) {
-    hly = GTY + 1; hlz = t - (GTZ + 2); hy = y0 + GTY; hz = z0 - 1 + hlz;
-  } else if (t < 2 * (GTZ + 2) + GTY) {
-    const int r = t - 2 * (GTZ + 2);
+  } else if (t < 2 * (TW + 2)) {
+    hly = TH + 1; hlz = t - (TW + 2); hy = y0 + TH; hz = z0 - 1 + hlz;
+  } else if (t < 2 * (TW + 2) + TH) {
+    const int r = t - 2 * (TW + 2);
     hly = r + 1; hlz = 0; hy = y0 + r; hz = z0 - 1;
-  } else if (t < 2 * (GTZ + 2) + 2 * GTY) {
-    const int r = t - 2 * (GTZ + 2) - GTY;
-    hly = r + 1; hlz = GTZ + 1; hy = y0 + r; hz = z0 + GTZ;
+  } else if (t < 2 * (TW + 2) + 2 * TH) {
+    const int r = t - 2 * (TW + 2) - TH;
+    hly = r + 1; hlz = TW + 1; hy = y0 + r; hz = z0 + TW;
   }
   const bool halo = hly >= 0;
 
   auto put = [&](int slot, const GRaw<F32> &own, const GRaw<F32> &hal, bool has_halo) {
     for (int q = 0; q < GNC; ++q) {
-      lds[slot][q][wave + 1][lane + 1] = own.value(q, DRIFT, cs, cu);
+      if (act) lds[slot][q][wave + 1][lane + 1] = own.value(q, DRIFT, cs, cu);
       if (has_halo) lds[slot][q][hly][hlz] = hal.value(q, DRIFT, cs, cu);
     }
   };
@@ -175,10 +195,9 @@ __global__ __launch_bounds__(64 * GTY) void k_gauge_tiled(const GaugePassArgs a,
   __syncthreads();
 
   double acc[5] = {0, 0, 0, 0, 0};
-  const int ly = wave + 1, lz = lane + 1;
-  for (int i = 0; i < XC; ++i) {
-    const int x = x0 + i;
-    const bool more = i + 1 < XC;
+  const int ly = y - y0 + 1, lz = z - z0 + 1;
+  for (int x = x0; x < xe; ++x) {
+    const bool more = x + 1 < xe;
     GRaw<F32> pown, phal;
     if (more) {
       pown.load(a, site(x + 2, y, z), u1, DRIFT);
@@ -218,10 +237,10 @@ __global__ __launch_bounds__(64 * GTY) void k_gauge_tiled(const GaugePassArgs a,
     g.Ad[2][1] = cur[3][ly - 1][lz + 1];
 
     const uint32_t s = site(x, y, z);
-    if (DRIFT) {
-      for (int q = 0; q < 2; ++q) nt_store_v<F32>(a.phi_out[q], a.philo_out[q], s, g.fc[q]);
+    if (DRIFT && act) {
+      for (int q = 0; q < 2; ++q) store_v<F32, !RAG>(a.phi_out[q], a.philo_out[q], s, g.fc[q]);
       if (u1)
-        for (int d = 0; d < 3; ++d) nt_store_v<F32>(a.A_out[d], a.Alo_out[d], s, g.Ac[d]);
+        for (int d = 0; d < 3; ++d) store_v<F32, !RAG>(a.A_out[d], a.Alo_out[d], s, g.Ac[d]);
     }
     P pin[2], pAin[3] = {0, 0, 0}, pout[2], pAout[3];
     if (KICK) {
@@ -237,13 +256,15 @@ __global__ __launch_bounds__(64 * GTY) void k_gauge_tiled(const GaugePassArgs a,
       gauge_site_f32<KICK, RED>(k, a.poly, g, pin, pAin, pout, pAout, acc);
     else
       gauge_site_f64<KICK, RED>(k, a.poly, g, pin, pAin, pout, pAout, acc);
-    if (KICK) {
-      for (int q = 0; q < 2; ++q) __builtin_nontemporal_store(pout[q], (P *)a.pi_out[q] + s);
+    if (KICK && act) {
+      for (int q = 0; q < 2; ++q) store_out<!RAG>((P *)a.pi_out[q] + s, pout[q]);
       if (u1)
-        for (int d = 0; d < 3; ++d) __builtin_nontemporal_store(pAout[d], (P *)a.piA_out[d] + s);
+        for (int d = 0; d < 3; ++d) store_out<!RAG>((P *)a.piA_out[d] + s, pAout[d]);
     }
-    if (RED && (i + 1) % RG == 0) {
+    if (RED && ((x + 1) % RG == 0 || (RAG && x + 1 == N))) {
       double v[kNumRed] = {0, 0, acc[2], acc[0], acc[1], acc[3], acc[4], 0};
+      if (!act)
+        for (int k2 = 2; k2 < 7; ++k2) v[k2] = 0.0;
       const size_t row = ((size_t)(x / RG) * nTy + ty) * nTz + tz;
       block_reduce_store_nt<kNumRed, 64 * GTY>(v, a.partials + row * kNumRed);
       for (int k2 = 0; k2 < 5; ++k2) acc[k2] = 0.0;
@@ -252,7 +273,7 @@ __global__ __launch_bounds__(64 * GTY) void k_gauge_tiled(const GaugePassArgs a,
       if (KICK) {
         for (int q = 0; q < GNC; ++q) pc[q] = pn[q];
         if (DRIFT) keep_p(pown, pn);
-        else if (i + 2 < XC) load_p(site(x + 2, y, z), pn);
+        else if (x + 2 < xe) load_p(site(x + 2, y, z), pn);
       }
       __syncthreads();  // every wavefront is done with slot sm (plane x - 1)
       put(sm, pown, phal, halo);  // plane x + 2 takes its slot
@@ -261,14 +282,14 @@ __global__ __launch_bounds__(64 * GTY) void k_gauge_tiled(const GaugePassArgs a,
   }
 }
 
-template <bool F32, int GTY, int U1 = 0>
+template <bool F32, int GTY, int U1 = 0, bool RAG = false>
 hipError_t dispatch_tiled(bool drift, bool kick, bool red, const GaugePassArgs &a, int blocks, int XC, hipStream_t s)
 {
   const int G = gauge_rows_g((int)a.N);
   const int code = (drift ? 4 : 0) | (kick ? 2 : 0) | (red ? 1 : 0);
 #define CLMI_GT(D, K, R)                                                                                  \
   case ((D ? 4 : 0) | (K ? 2 : 0) | (R ? 1 : 0)):                                                        \
-    hipLaunchKernelGGL((k_gauge_tiled<F32, D, K, R, GTY, U1>), dim3(blocks), dim3(64 * GTY), 0, s, a, XC, G); \
+    hipLaunchKernelGGL((k_gauge_tiled<F32, D, K, R, GTY, U1, RAG>), dim3(blocks), dim3(64 * GTY), 0, s, a, XC, G); \
     break;
   switch (code) {
     CLMI_GT(true, true, true)
@@ -287,26 +308,46 @@ hipError_t dispatch_tiled(bool drift, bool kick, bool red, const GaugePassArgs &
 
 }  // namespace
 
-// Shape of the tiled pass with TY-row tiles (4 or 8) and x-chunk XC (a power of two dividing N, a multiple
-// of the row group G): workgroups and partial-sum rows; false when N does not fit the tile.
+// Shape of the tiled pass with TY-row tiles (4 or 8) and x-chunk XC (a multiple of the row group G, and a power of
+// two that divides N where N is a multiple of 64): workgroups and partial-sum rows; false when N does not fit the tile.
 bool gauge_tiled_shape(int N, int ty, int XC, int *blocks, int *rows)
 {
-  if ((ty != 4 && ty != 8) || N % GTZ != 0 || N % ty != 0) return false;
+  if ((ty != 4 && ty != 8) || (N & 1)) return false;
+  const bool rag = N % GTZ != 0;
+  if (rag && (ty != 4 || !gauge_ragged(N))) return false;
   const int G = gauge_rows_g(N);
-  if (XC < G || XC > N || N % XC != 0 || XC % G != 0 || (XC & (XC - 1)) != 0) return false;
-  const long tiles = (long)(N / ty) * (N / GTZ);
-  *blocks = (int)(tiles * (N / XC));
-  *rows = (int)(tiles * (N / G));
+  if (XC < G || XC > (rag ? N + G : N) || XC % G != 0) return false;
+  if (!rag && (N % XC != 0 || (XC & (XC - 1)) != 0)) return false;
+  const long tiles = (long)((N + ty - 1) / ty) * ((N + GTZ - 1) / GTZ);
+  *blocks = (int)(tiles * ((N + XC - 1) / XC));
+  *rows = (int)(tiles * ((N + G - 1) / G));
   return true;
 }
 
 // Default plan: the longest x-chunk that still gives every CU two workgroups (two 4-wave workgroups
 // fill a CU at the pass's two waves per SIMD), else the shortest; longer chunks re-read fewer x-halo
 // planes.  Measured at 256^3: XC 16 -> 128 takes the pass from 706 to 652 us (FP64) and 546 to 475 us
-// (FP32-bulk).
+// (FP32-bulk).  For N no multiple of 64 the tiles seldom fill the 2 ncu places, and a power of two seldom divides N:
+// there the x-chunk with the least (rounds of 2 ncu workgroups) x (its planes + 3 of start-up), the time of a
+// plane being much the same in every round: 200^3 FP64 takes 40 planes (1000 workgroups, two rounds) and not 64.
 bool gauge_tiled_plan(int N, int ty, int ncu, int *XC, int *blocks, int *rows)
 {
   int best = 0;
+  if (N % GTZ != 0) {
+    long least = 0;
+    for (int xc = gauge_rows_g(N); xc < N + gauge_rows_g(N); xc += gauge_rows_g(N)) {
+      int b = 0, r = 0;
+      if (!gauge_tiled_shape(N, ty, xc, &b, &r)) continue;
+      const long cost = (long)((b + 2 * ncu - 1) / (2 * ncu)) * (xc + 3);
+      if (best == 0 || cost < least) {
+        best = xc;
+        least = cost;
+      }
+    }
+    if (best == 0) return false;
+    *XC = best;
+    return gauge_tiled_shape(N, ty, best, blocks, rows);
+  }
   for (int xc = 8; xc <= N; xc *= 2) {
     int b = 0, r = 0;
     if (!gauge_tiled_shape(N, ty, xc, &b, &r)) continue;
@@ -321,6 +362,10 @@ hipError_t launch_gauge_tiled(bool f32, int ty, bool drift, bool kick, bool red,
                               int XC, hipStream_t s)
 {
   const bool u1 = a.has_u1 != 0;
+  if (a.N % GTZ != 0)
+    return f32 ? (u1 ? dispatch_tiled<true, 4, 1, true>(drift, kick, red, a, blocks, XC, s)
+                     : dispatch_tiled<true, 4, 0, true>(drift, kick, red, a, blocks, XC, s))
+               : dispatch_tiled<false, 4, 0, true>(drift, kick, red, a, blocks, XC, s);
   if (ty == 8)
     return f32 ? (u1 ? dispatch_tiled<true, 8, 1>(drift, kick, red, a, blocks, XC, s)
                      : dispatch_tiled<true, 8>(drift, kick, red, a, blocks, XC, s))

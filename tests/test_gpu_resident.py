@@ -7,8 +7,8 @@ import threading
 import numpy as np
 import pytest
 
-from cosmolattice_amd.clmi import (CLMI_F32_BULK, CLMI_F64, CLMI_FLAG_NO_TILED, FLD_S, PI_S, PV_WEIGHTS, VV_WEIGHTS,
-                                   Lattice, lphi4)
+from cosmolattice_amd.clmi import (CLMI_F32_BULK, CLMI_F64, CLMI_FLAG_NO_TILED, FLD_CS, FLD_S, FLD_U1, PI_CS, PI_S,
+                                   PI_U1, PV_WEIGHTS, VV_WEIGHTS, Lattice, lphi4, lphi4U1)
 
 pytestmark = pytest.mark.gpu
 
@@ -114,6 +114,44 @@ def test_ragged_sides_bit_identical_to_one_site_per_thread(gpu, N, prec, kind, s
         for k in ("pi2S", "grad2S", "pot"):
             assert sums[k] == pytest.approx(res[0][1][k], rel=1e-13)
     assert res[1][1] == res[2][1]
+
+
+U1_KINDS = [(FLD_CS, 0), (FLD_CS, 1), (PI_CS, 0), (PI_CS, 1)] + [(k, d) for k in (FLD_U1, PI_U1) for d in range(3)]
+
+
+# tile edges: one short row tile (52, 62), two of 38 sites and a last tile of rows that is full (76), a short last tile of
+# rows and x-chunk (90, 130)
+@pytest.mark.parametrize("N", [52, 62, 76, 90, 130])
+@pytest.mark.parametrize("prec", [CLMI_F64, CLMI_F32_BULK])
+@pytest.mark.parametrize("scheme", ["LF", "VV2", "PV2"])
+def test_ragged_u1_bit_identical_to_one_site_per_thread(gpu, N, prec, scheme):
+    """The tiled charged-scalar + U(1) pass on a side that is no multiple of 64, static background: every array equals
+    the one-site-per-thread pass's to the bit; its sums differ in order only."""
+    print(f"case ragged u1 N={N} prec={prec} {scheme}", flush=True)
+    spec = lphi4U1(10.0, phi0_gev=5.6964e18, lam=1.0, pi0_gev2=0.0)
+    rng = np.random.default_rng(N)
+    ics = {kc: 0.3 * rng.standard_normal((N, N, N)) for kc in U1_KINDS}
+    res = []
+    for flags, kernel in ((CLMI_FLAG_NO_TILED, "k_gauge_pass"), (0, "k_gauge_tiled")):
+        lat = Lattice(spec, N, 0.4909, 0.005, prec, expansion=False, flags=flags)
+        assert lat.plan().split()[0] == kernel
+        for (k, c), a in ics.items():
+            lat.upload(k, 0, c, a)
+        lat.set_background(aI=1.1, aSI=1.05, aIM=1.0)
+        if scheme == "LF":
+            lat.lf_init()
+            lat.lf_evolve(3)
+            lat.lf_sync()
+        elif scheme == "VV2":
+            lat.vv_evolve([1.0], 2)
+        else:
+            lat.pv_evolve([1.0], 2)
+        res.append(([lat.download(k, 0, c) for k, c in ics], lat.averages()))
+        lat.close()
+    for a, b in zip(res[0][0], res[1][0]):
+        assert np.array_equal(a, b)
+    for k in ("pi2CS", "grad2CS", "pot", "pi2U1", "B2U1"):
+        assert res[1][1][k] == pytest.approx(res[0][1][k], rel=1e-13)
 
 
 def test_resident_two_threads(gpu):
