@@ -27,7 +27,7 @@ __global__ __launch_bounds__(kUpdThreads) void k_update(DevState *st, const doub
   double red[kNumRed];
   for (int k = 0; k < kNumRed; ++k) red[k] = rows > 0 ? tot[k] * mc.invV : s.red[k];
   for (int k = 0; k < kNumRed; ++k) s.red[k] = red[k];
-  apply_update(&s, red, mc, ops);
+  apply_update<false>(&s, red, mc, ops);
   *st = s;
 }
 
@@ -50,7 +50,7 @@ __global__ __launch_bounds__(kUpdThreads) void k_update_batch(const UpdMember *m
   double red[kNumRed];
   for (int k = 0; k < kNumRed; ++k) red[k] = u.rows > 0 ? tot[k] * mc.invV : s.red[k];
   for (int k = 0; k < kNumRed; ++k) s.red[k] = red[k];
-  apply_update(&s, red, mc, ops);
+  apply_update<false>(&s, red, mc, ops);
   *u.st = s;
 }
 

@@ -47,6 +47,8 @@ struct clmi_ctx {
   DevState *dstate = nullptr;
   double *partials = nullptr;
   double *dscratch = nullptr;  // small device scratch for row sums
+  unsigned *done_count = nullptr;  // workgroups of the running pass that have finished (pass_tail.hpp)
+  bool tail_ok = false;            // integer alpha: the update may run in the pass's last workgroup
   int blocks_s = 0, blocks_g = 0;
   int rows_g = 0;  // partial-sum rows a reducing charged-scalar + U(1) pass writes
   clmi_background *snap = nullptr;  // device target of the next storeFieldsAverages snapshot (adjoint tape)
@@ -273,16 +275,29 @@ GaugePassArgs gauge_args(const clmi_ctx *c, int fi, int fo, int pi, int po, doub
 }
 
 // Launch one lattice pass over every sector; returns the number of partial rows written in *rows.
+// ops (reducing passes): run this background update in the pass's last workgroup; *updated says whether it does.  The
+// scalar-singlet full-row and plane-chunk passes do (what it gains: pass_tail.hpp), but for a pass that is timed by
+// itself and a model whose update needs the general power.
 // ckick2_s != 0 (drift + kick passes of scalar-singlet models on the full-row pass): kick the scalars a
 // second time, by ckick2_s, from the same drifted fields (see double_kick_ok).
 int run_pass(clmi_ctx *c, bool drift, bool kick, bool red, double cdt_s, double ckick_s, double ckick_g, int *rows,
-             double ckick2_s = 0.0)
+             double ckick2_s = 0.0, const UpdateOps *ops = nullptr, bool *updated = nullptr)
 {
   const bool kick2 = ckick2_s != 0.0;
   if (kick2 && !(drift && kick && (c->rowk || c->tiled || c->flat) && c->cfg.n_cscalars == 0))
     return fail(c, CLMI_E_INVALID, "double kick outside a scalar-singlet full-row, tiled or plane-chunk drift + kick pass");
   const bool timed = c->prof && drift && kick && (c->prof_count++ % c->prof_every == 0);
   if (timed) CHK(prof_event(c));
+  PassTail tail{};
+  if (ops && red && c->tail_ok && !timed && (c->rowk || c->flat) && c->cfg.n_cscalars == 0) {
+    tail.on = 1;
+    tail.partials = c->partials;
+    tail.st = c->dstate;
+    tail.count = c->done_count;
+    tail.mc = c->mc;
+    tail.ops = *ops;
+  }
+  if (updated) *updated = tail.on != 0;
   int r = 0;
   if (c->cfg.n_scalars > 0) {
     const int fi = c->cur_fS, fo = drift ? 1 - c->cur_fS : c->cur_fS;
@@ -292,6 +307,8 @@ int run_pass(clmi_ctx *c, bool drift, bool kick, bool red, double cdt_s, double 
     const int nrows = c->rowk ? c->rplan.rows : c->tiled ? c->tplan.rows : c->flat ? c->fplan.rows : c->blocks_s;
     if (red && (size_t)r + nrows > c->partial_rows)
       return fail(c, CLMI_E_INVALID, "partial-sum buffer too small for the scalar pass");
+    a.tail = tail;
+    a.tail.rows = nrows;
     if (c->rowk) {
       HIPCHK(c, launch_scalar_rows(c->cfg.n_scalars, c->f32, drift, kick, red, a, c->rplan, c->stream, kick2));
       if (red) r += c->rplan.rows;
@@ -351,15 +368,14 @@ int pass_update(clmi_ctx *c, bool drift, bool kick, bool red, double cdt_s, doub
                 bool do_update, std::initializer_list<std::pair<int, double>> ops, double ckick2_s = 0.0)
 {
   int rows = 0;
-  CHK(run_pass(c, drift, kick, red, cdt_s, ckick_s, ckick_g, &rows, ckick2_s));
-  if (do_update) {
-    UpdateOps u = make_ops(ops);
-    if (c->snap && u.n > 0 && u.op[0] == OP_STORE_FIELDS) {
-      u.snap = c->snap;
-      c->snap = nullptr;
-    }
-    HIPCHK(c, launch_update(c->dstate, c->partials, rows, c->mc, u, c->stream));
+  bool updated = false;
+  UpdateOps u = make_ops(ops);
+  if (do_update && c->snap && u.n > 0 && u.op[0] == OP_STORE_FIELDS) {
+    u.snap = c->snap;
+    c->snap = nullptr;
   }
+  CHK(run_pass(c, drift, kick, red, cdt_s, ckick_s, ckick_g, &rows, ckick2_s, do_update ? &u : nullptr, &updated));
+  if (do_update && !updated) HIPCHK(c, launch_update(c->dstate, c->partials, rows, c->mc, u, c->stream));
   return CLMI_OK;
 }
 
@@ -645,6 +661,7 @@ int clmi_create(const clmi_config *cfg, clmi_ctx **out)
   c->partial_rows = rows;
   if (hipMalloc(&c->partials, rows * kNumRed * sizeof(double)) != hipSuccess ||
       hipMalloc(&c->dscratch, 64 * sizeof(double)) != hipSuccess ||
+      hipMalloc(&c->done_count, sizeof(unsigned)) != hipSuccess ||
       hipMalloc(&c->dstate, sizeof(DevState)) != hipSuccess) {
     fail(c, CLMI_E_NOMEM, "device allocation failed");
     return bail(CLMI_E_NOMEM);
@@ -671,8 +688,14 @@ int clmi_create(const clmi_config *cfg, clmi_ctx **out)
   c->mc.MPl = g.MPl;
   c->mc.invV = 1.0 / ((double)g.N * g.N * g.N);
 
+  c->tail_ok = g.alpha == std::rint(g.alpha) && std::fabs(g.alpha) <= 15.0;
+
   DevState h{};
   h.bg.aI = h.bg.aSI = h.bg.aIM = 1.0;
+  if (hipMemsetAsync(c->done_count, 0, sizeof(unsigned), c->stream) != hipSuccess) {
+    fail(c, CLMI_E_HIP, "counter initialisation failed");
+    return bail(CLMI_E_HIP);
+  }
   if (hipMemcpyAsync(c->dstate, &h, sizeof(DevState), hipMemcpyHostToDevice, c->stream) != hipSuccess) {
     fail(c, CLMI_E_HIP, "state upload failed");
     return bail(CLMI_E_HIP);
@@ -704,6 +727,7 @@ void clmi_destroy(clmi_ctx *c)
     }
   if (c->partials) (void)hipFree(c->partials);
   if (c->dscratch) (void)hipFree(c->dscratch);
+  if (c->done_count) (void)hipFree(c->done_count);
   if (c->res_lines) (void)hipFree(c->res_lines);
   if (c->res_xch) (void)hipFree(c->res_xch);
   if (c->res_err) (void)hipHostFree(c->res_err);

@@ -103,6 +103,16 @@ struct DevArr {
   float *lo = nullptr; // F32 bulk fields: low word; nullptr for momenta / F64
 };
 
+// Background update run by the last workgroup of a reducing full-row or plane-chunk pass (pass_tail.hpp); on = 0: none.
+struct PassTail {
+  int on, rows;            // partial rows of the pass
+  const double *partials;
+  DevState *st;
+  unsigned *count;         // workgroups that have finished; 0 between passes
+  ModelConsts mc;
+  UpdateOps ops;
+};
+
 struct ScalarPassArgs {
   const void *phi_in[CLMI_MAX_SCALARS];
   const float *philo_in[CLMI_MAX_SCALARS];
@@ -120,6 +130,7 @@ struct ScalarPassArgs {
   const DevState *st;
   double *partials;  // this pass's rows, kNumRed doubles each
   ScalarPoly poly;
+  PassTail tail;
 };
 
 struct GaugePassArgs {
@@ -181,6 +192,14 @@ __device__ __forceinline__ double wave_sum(double v)
   return v;
 }
 
+// Slot threadIdx.x of a partial row, through the coherence point: the workgroup that finishes a pass reads the rows
+// of all others within the launch.
+__device__ __forceinline__ void store_row(double *row, double s)
+{
+  __hip_atomic_store((uint64_t *)row + threadIdx.x, __builtin_bit_cast(uint64_t, s), __ATOMIC_RELAXED,
+                     __HIP_MEMORY_SCOPE_AGENT);
+}
+
 // Deterministic block reduction: wavefront sums, then a fixed-order sum over the block's
 // wavefronts; thread k < K writes slot k of the block's row.
 // Sum of v over a block of NTB threads, stored by threads 0..K-1 into row[0..K).
@@ -199,7 +218,7 @@ __device__ __forceinline__ void block_reduce_store_nt(double (&v)[K], double *ro
     double s = 0.0;
 #pragma unroll
     for (int w = 0; w < NTB / 64; ++w) s += sh[w][threadIdx.x];
-    row[threadIdx.x] = s;
+    store_row(row, s);
   }
 }
 

@@ -203,6 +203,7 @@ __global__ __launch_bounds__(kFlatThreads) void k_scalar_flat(const ScalarPassAr
       __syncthreads();
     }
   }
+  if constexpr (RED) finish_pass<NTH>(a.tail);
 }
 
 template <int NF, bool F32, int VZ, int NH, int PK>

@@ -17,6 +17,7 @@
 #pragma once
 
 #include "clmi_internal.hpp"
+#include "pass_tail.hpp"
 #include "scalar_poly.hpp"
 
 namespace clmi {
@@ -182,7 +183,7 @@ __device__ __forceinline__ void block_reduce_rows(double (&v)[K], double *row)
     double s = 0.0;
 #pragma unroll
     for (int w = 0; w < NW; ++w) s += sh[w][threadIdx.x];
-    row[threadIdx.x] = s;
+    store_row(row, s);
   }
 }
 
@@ -450,6 +451,7 @@ __global__ __launch_bounds__(64 * WPR * TY) void k_scalar_rows(const ScalarPassA
 {
   __shared__ RowsTile<NF, F32, VZ, WPR, TY> ldsbuf;
   rows_body<NF, F32, VZ, WPR, TY, DRIFT, KICK, RED, MM, PK, KICK2>(a, XC, G, blockIdx.x, gridDim.x, ldsbuf);
+  if constexpr (RED) finish_pass<64 * WPR * TY>(a.tail);
 }
 
 // kick2: the double-kick form of the drift + kick pass.

@@ -52,13 +52,6 @@ __device__ __forceinline__ double sf_kernel_of(double a, double pi2S, double gra
           (mc.alpha + 1) * pot);
 }
 
-// ScaleFactorKernels::get: integer-time averages.
-template <bool INT>
-__device__ __forceinline__ double sf_kernel(const clmi_background &b, const ModelConsts &mc)
-{
-  return sf_kernel_of<INT>(b.aI, b.pi2AvI, b.grad2AvI, b.CSpi2AvI, b.CSgrad2AvI, b.U1pi2AvI, b.U1Mag2AvI, b.potAvI, mc);
-}
-
 // Fixed-order sum of `rows` partial rows by a block of NT threads: thread t adds rows t, t + NT, ... in
 // that order, four rows in flight per batch (each row one 64-byte line, read as four 16-byte loads),
 // then wavefront sums, then those in order.  Result in out[0..kNumRed)
@@ -109,12 +102,16 @@ __device__ inline void sum_partials(const double *partials, int rows, double *ou
 
 // One background operation (UpdateOp), executed by one thread.  red: finished volume averages (sums / N^3) of
 // the last pass.  a_drift > 0: the drift coefficients use this scale factor instead of aSI.
+// Averages first, then one evaluation of the scale-factor kernel for every operation that needs it, then what it
+// moves: this is compiled into every reducing pass (pass_tail.hpp), and seven copies of the kernel were 4 KB of it.
 template <bool INT>
 __device__ __forceinline__ void apply_op(DevState *st, const double *red, const ModelConsts &mc, const int op,
                                          const double w, double &a_drift)
 {
   clmi_background &b = st->bg;
   const double dt = mc.dt;
+  bool kernel = false;
+  double g2 = b.grad2AvI, cg2 = b.CSgrad2AvI, b2 = b.U1Mag2AvI;  // the kernel's averages, where not the integer-time ones
   switch (op) {
     case OP_STORE_FIELDS:  // leapfrog.h:269-277
       if (mc.ns > 0) b.grad2AvI = red[RED_GRAD2S];
@@ -122,7 +119,7 @@ __device__ __forceinline__ void apply_op(DevState *st, const double *red, const 
       if (mc.nu1 > 0) b.U1Mag2AvI = red[RED_B2U1];
       b.potAvI = red[RED_POT];
       break;
-    case OP_LF_MOMENTA:  // leapfrog.h:239-267 then 124-129 and 168-184
+    case OP_LF_MOMENTA:  // leapfrog.h:239-267
       if (mc.ns > 0) {
         b.pi2AvSIM = b.pi2AvSI;
         b.pi2AvSI = red[RED_PI2S];
@@ -138,33 +135,21 @@ __device__ __forceinline__ void apply_op(DevState *st, const double *red, const 
         b.U1pi2AvSI = red[RED_PI2U1];
         b.U1pi2AvI = 0.5 * (b.U1pi2AvSIM + b.U1pi2AvSI);
       }
-      st->K = sf_kernel<INT>(b, mc);
-      b.aDotSIM = b.aDotSI;
-      b.aDotSI += dt * st->K;
-      b.aDotI = (b.aDotSIM + b.aDotSI) / 2.0;
-      b.aIM = b.aI;
-      b.aI += dt * b.aDotSI;
-      b.aSI = (b.aIM + b.aI) / 2.0;
+      kernel = true;
       break;
     case OP_LF_SYNC:  // leapfrog.h:105-112
-      if (mc.ns > 0) b.pi2AvI = red[RED_PI2S];
-      if (mc.ncs > 0) b.CSpi2AvI = red[RED_PI2CS];
-      if (mc.nu1 > 0) b.U1pi2AvI = red[RED_PI2U1];
-      st->K = sf_kernel<INT>(b, mc);
-      b.aDotI = b.aDotSI + dt / 2.0 * st->K;
-      break;
-    case OP_LF_INIT:  // leapfrog.h:35
-      st->K = sf_kernel<INT>(b, mc);
-      b.aDotSI = b.aDotI - dt / 2.0 * st->K;
-      break;
-    case OP_VV_SF_HALF:  // velocityverlet.h:165-168
-      st->K = sf_kernel<INT>(b, mc);
-      b.aDotSI = b.aDotI + (dt / 2) * st->K * w;
-      break;
+      kernel = true;
+      [[fallthrough]];
     case OP_VV_MOMENTA:  // velocityverlet.h:249-256
       if (mc.ns > 0) b.pi2AvI = red[RED_PI2S];
       if (mc.ncs > 0) b.CSpi2AvI = red[RED_PI2CS];
       if (mc.nu1 > 0) b.U1pi2AvI = red[RED_PI2U1];
+      break;
+    case OP_LF_INIT:      // leapfrog.h:35
+    case OP_VV_SF_HALF:   // velocityverlet.h:165-168
+    case OP_VV_SF_ONE:    // velocityverlet.h:171-174
+    case OP_KERNEL_ONLY:
+      kernel = true;
       break;
     case OP_VV_MOMENTA_KICK2:  // velocityverlet.h:249-256, scalar singlets only
       b.pi2AvI = red[RED_PI2S_KICK2];
@@ -173,10 +158,6 @@ __device__ __forceinline__ void apply_op(DevState *st, const double *red, const 
       b.aIM = b.aI;
       b.aI += dt * b.aDotSI * w;
       b.aSI = (b.aIM + b.aI) / 2.0;
-      break;
-    case OP_VV_SF_ONE:  // velocityverlet.h:171-174
-      st->K = sf_kernel<INT>(b, mc);
-      b.aDotI = b.aDotSI + (dt / 2) * st->K * w;
       break;
     case OP_SET_ALL:  // averages.h:86-116
       b.potAvI = red[RED_POT];
@@ -197,9 +178,6 @@ __device__ __forceinline__ void apply_op(DevState *st, const double *red, const 
         b.CSgrad2AvI = red[RED_GRAD2CS];
       }
       break;
-    case OP_KERNEL_ONLY:
-      st->K = sf_kernel<INT>(b, mc);
-      break;
     case OP_PV_SF_FIRST:  // positionverlet.h:196-209; the first drift of the stage uses aI before it
       a_drift = b.aI;
       b.aIM = b.aI;
@@ -208,7 +186,7 @@ __device__ __forceinline__ void apply_op(DevState *st, const double *red, const 
       break;
     case OP_PV_MID: {  // positionverlet.h:73-94
       // storeFieldsAveragesHalf (positionverlet.h:258-266): the half-step field averages feed getSI
-      const double g2SI = red[RED_GRAD2S], cg2SI = red[RED_GRAD2CS], b2SI = red[RED_B2U1];
+      g2 = red[RED_GRAD2S], cg2 = red[RED_GRAD2CS], b2 = red[RED_B2U1];
       b.potAvSI = red[RED_POT];
       // storeMomentaAverages (positionverlet.h:238-256)
       const double pIM = b.pi2AvI, cIM = b.CSpi2AvI, uIM = b.U1pi2AvI;
@@ -218,16 +196,46 @@ __device__ __forceinline__ void apply_op(DevState *st, const double *red, const 
       b.pi2AvSI = 0.5 * (b.pi2AvI + pIM);
       b.CSpi2AvSI = 0.5 * (b.CSpi2AvI + cIM);
       b.U1pi2AvSI = 0.5 * (b.U1pi2AvI + uIM);
-      // kickScaleFactor with ScaleFactorKernels::getSI (positionverlet.h:151-154)
-      st->K = sf_kernel_of<INT>(b.aI, b.pi2AvSI, g2SI, b.CSpi2AvSI, cg2SI, b.U1pi2AvSI, b2SI, b.potAvSI, mc);
-      b.aDotI += dt * st->K * w;
-      // driftScaleFactorSecondHalf (positionverlet.h:212-223); the second drift uses the new aI
-      b.aI += dt / 2.0 * b.aDotI * w;
-      b.aSI = (b.aIM + b.aI) / 2.0;
-      a_drift = b.aI;
+      kernel = true;
       break;
     }
     case OP_PV_DRIFT_AI:
+      a_drift = b.aI;
+      break;
+    default:
+      break;
+  }
+  if (!kernel) return;
+  const bool si = op == OP_PV_MID;  // ScaleFactorKernels::getSI (positionverlet.h:151-154), else ::get
+  const double K = sf_kernel_of<INT>(b.aI, si ? b.pi2AvSI : b.pi2AvI, g2, si ? b.CSpi2AvSI : b.CSpi2AvI, cg2,
+                                     si ? b.U1pi2AvSI : b.U1pi2AvI, b2, si ? b.potAvSI : b.potAvI, mc);
+  st->K = K;
+  switch (op) {
+    case OP_LF_MOMENTA:  // leapfrog.h:124-129 and 168-184
+      b.aDotSIM = b.aDotSI;
+      b.aDotSI += dt * K;
+      b.aDotI = (b.aDotSIM + b.aDotSI) / 2.0;
+      b.aIM = b.aI;
+      b.aI += dt * b.aDotSI;
+      b.aSI = (b.aIM + b.aI) / 2.0;
+      break;
+    case OP_LF_SYNC:
+      b.aDotI = b.aDotSI + dt / 2.0 * K;
+      break;
+    case OP_LF_INIT:
+      b.aDotSI = b.aDotI - dt / 2.0 * K;
+      break;
+    case OP_VV_SF_HALF:
+      b.aDotSI = b.aDotI + (dt / 2) * K * w;
+      break;
+    case OP_VV_SF_ONE:
+      b.aDotI = b.aDotSI + (dt / 2) * K * w;
+      break;
+    case OP_PV_MID:
+      b.aDotI += dt * K * w;
+      // driftScaleFactorSecondHalf (positionverlet.h:212-223); the second drift uses the new aI
+      b.aI += dt / 2.0 * b.aDotI * w;
+      b.aSI = (b.aIM + b.aI) / 2.0;
       a_drift = b.aI;
       break;
     default:
@@ -253,14 +261,15 @@ __device__ __forceinline__ void refresh_coefficients(DevState *st, const ModelCo
 }
 
 // Executed by one thread: the operations in order, then the coefficients.
-__device__ inline void apply_update(DevState *st, const double *red, const ModelConsts &mc, const UpdateOps &ops)
+template <bool INT>
+__device__ __forceinline__ void apply_update(DevState *st, const double *red, const ModelConsts &mc, const UpdateOps &ops)
 {
   double a_drift = -1.0;
   for (int o = 0; o < ops.n; ++o) {
-    apply_op<false>(st, red, mc, ops.op[o], ops.w[o], a_drift);
+    apply_op<INT>(st, red, mc, ops.op[o], ops.w[o], a_drift);
     if (o == 0 && ops.snap) *ops.snap = st->bg;
   }
-  refresh_coefficients<false>(st, mc, a_drift);
+  refresh_coefficients<INT>(st, mc, a_drift);
 }
 
 }  // namespace clmi
