@@ -138,8 +138,13 @@ int fail(clmi_ctx *c, int code, const std::string &msg)
 size_t bytes_field(bool f32) { return f32 ? 4 : 8; }
 
 // Row-pass shape selector from clmi_config.flags (bit 0: VZ = 4 rows, bit 1: 4-row tiles).
-// Memory mode of the full-row pass when neither the configuration nor clmi_autotune chooses one.
-constexpr int kDefaultMemMode = 15;
+// Memory mode of the full-row pass when neither the configuration nor clmi_autotune chooses one, for a state of `bytes` in
+// both of its buffers: ordinary accesses where it stays in the 256 MB last-level cache from step to step, else
+// non-temporal stores.  A leapfrog step, modes 0 / 1 / 15: 128^3 two fields FP32-bulk (100 MB) 24.1 / 30.0 / 31.0 us and
+// FP64 (134 MB) 27.8 / 32.5 / 33.9, 192^3 one field FP64 (226 MB) 43.5 / 56 / 61; past the cache 192^3 two fields
+// FP32-bulk (340 MB) 86.5 / 82.7 / 84.4 and FP64 (453 MB) 124 / 112 / 123, 256^3 FP32-bulk 181 / 177 / 174, 512^3 - / 1457 /
+// 1510 to 1700.
+int default_mem_mode(double bytes) { return bytes <= 256.0 * 1048576.0 ? 0 : 1; }
 
 int rows_shape(int flags)
 {
@@ -678,25 +683,33 @@ int clmi_create(const clmi_config *cfg, clmi_ctx **out)
   c->blocks_g = gauge_pass_blocks(c->V);
   c->rows_g = c->blocks_g;
   if (!(g.flags & CLMI_FLAG_NO_TILED)) {
-    // Default x-chunk of the full-row pass: the longest of 32, 16, 8 that still gives every CU a
-    // workgroup, else the shortest (small lattices).  clmi_autotune refines it; results do not depend on it.
+    // Default x-chunk of the full-row pass: the least (rounds of ncu workgroups) x (planes of a chunk + 2 of start-up),
+    // since a workgroup takes a CU to itself (512 threads of more than 128 registers, or 1024) and a plane takes much
+    // the same time in every round; among equals the longer.  192^3, two fields: 24 (192 workgroups, one round of 26
+    // planes) 84 us FP32-bulk and 123 us FP64, 16 (288, two rounds of 18) 104 and 157, 8 92 and 136, 32 100 and 152;
+    // 256^3 FP32-bulk 32 173, 16 175, 64 250; 512^3 64 1560, 32 1690.  clmi_autotune refines it; results do not depend
+    // on it.
     int ncu = 0;
     if (hipDeviceGetAttribute(&ncu, hipDeviceAttributeMultiprocessorCount, c->device) != hipSuccess || ncu < 1)
       ncu = 256;
     RowsPlan rp;
-    const int mm_req = (g.flags >> 8) & 15;
+    const int mm_req = (g.flags >> 8) & 15, mm_def = default_mem_mode(fused_pass_bytes(c));
     // FP64 at 256^3: the full-row pass needs 1024-thread workgroups, whose 128-VGPR cap makes it spill, and
     // the tiled pass is faster there.  Batched ensembles stop at 192^3, so nothing needs the row plan.  A
     // memory-mode or shape flag still asks for the full-row pass.
     const bool asked = mm_req != 0 || (g.flags & (CLMI_FLAG_SHAPE_ALT | CLMI_FLAG_SHAPE_TY4)) != 0;
     const bool prefer_tiled = g.precision == CLMI_F64 && g.N == 256 && !asked;
-    for (int xc : {32, 16, 8})
+    long least = 0;
+    for (int xc : {64, 32, 24, 16, 8})
       if (!prefer_tiled &&
-          scalar_rows_plan(g.N, g.n_scalars, g.precision == CLMI_F32_BULK, xc, mm_req ? mm_req : kDefaultMemMode,
+          scalar_rows_plan(g.N, g.n_scalars, g.precision == CLMI_F32_BULK, xc, mm_req ? mm_req : mm_def,
                            rows_shape(g.flags), &rp)) {
+        const long cost = (long)((rp.blocks + ncu - 1) / ncu) * (xc + 2);
+        if (!c->rowk || cost < least) {
+          c->rplan = rp;
+          least = cost;
+        }
         c->rowk = true;
-        c->rplan = rp;
-        if (rp.blocks >= ncu) break;
       }
     if (mm_req && !c->rowk) {
       fail(c, CLMI_E_INVALID, "memory mode " + std::to_string(mm_req) + " is not available for this lattice");
@@ -1912,6 +1925,7 @@ struct clmi_ensemble {
   int nf = 0;
   int pk = 0;  // potential form of the batched passes (1: every member has the compile-time lphi4 table)
   bool f32 = false, ex = false;
+  int mm = 1;  // memory mode of the batched passes (default_mem_mode of all members together)
   std::string err;
 };
 
@@ -2011,7 +2025,7 @@ int ens_tables(clmi_ensemble *e)
 // One steady-state leapfrog step of a group: fused drift+kick pass, then the background update.
 int ens_step(clmi_ensemble *e, const clmi_ensemble::Group &g, int parity, hipStream_t st)
 {
-  EHIP(e, launch_scalar_rows_batch(e->nf, e->f32, e->pk, g.vz, true, true, e->ex, e->d_rows[parity] + g.first, g.count,
+  EHIP(e, launch_scalar_rows_batch(e->nf, e->f32, e->pk, e->mm, g.vz, true, true, e->ex, e->d_rows[parity] + g.first, g.count,
                                    g.blocks, st));
   if (e->ex)
     EHIP(e, launch_update_batch(e->d_upd + g.first, g.count,
@@ -2081,6 +2095,9 @@ int clmi_ensemble_create(clmi_ctx *const *members, int n, size_t group_bytes, cl
   e->pk = 1;  // the batched shapes are the 512-thread ones, where both precisions use it
   for (clmi_ctx *c : e->m)
     if (poly_kind(c->spoly, e->nf) != 1) e->pk = 0;
+  double state = 0.0;
+  for (clmi_ctx *c : e->m) state += fused_pass_bytes(c);
+  e->mm = default_mem_mode(state);
   e->ex = c0->cfg.expansion != 0;
   e->group_bytes = group_bytes ? group_bytes : SIZE_MAX;
   int rc = CLMI_OK;
@@ -2152,7 +2169,7 @@ int clmi_ensemble_autotune(clmi_ensemble *e, int reps, char *report, size_t repo
       if ((rc = ens_tables(e)) != CLMI_OK) break;
       const clmi_ensemble::Group &g = e->groups[gi];
       auto launch = [&]() {
-        return launch_scalar_rows_batch(e->nf, e->f32, e->pk, g.vz, true, true, e->ex, e->d_rows[0] + g.first, g.count,
+        return launch_scalar_rows_batch(e->nf, e->f32, e->pk, e->mm, g.vz, true, true, e->ex, e->d_rows[0] + g.first, g.count,
                                         g.blocks, e->stream);
       };
       hipError_t he = launch();
@@ -2252,7 +2269,7 @@ int autotune_gauge(clmi_ctx *c, int reps, std::string &rep)
   int best_xc = c->gXC, best_blocks = c->blocks_g;
   std::string lines;
   hipError_t e = hipSuccess;
-  for (int xc = 8; xc <= c->N && e == hipSuccess; xc *= 2) {
+  for (int xc = 4; xc <= c->N && e == hipSuccess; xc *= 2) {
     int blocks = 0, rows = 0;
     if (!gauge_tiled_shape(c->N, c->gTY, xc, &blocks, &rows) || rows != c->rows_g) continue;
     auto launch = [&]() { return launch_gauge_tiled(c->f32, c->gTY, true, true, true, a, blocks, xc, c->stream); };
@@ -2319,10 +2336,13 @@ int clmi_autotune(clmi_ctx *c, int reps, char *report, size_t report_len)
   int rc = CLMI_OK;
   // row kernel: memory modes 1 (NT stores), 3 (+ NT momentum loads), 7 (+ NT loads of own field rows),
   // 15 (as 7, but ordinary loads for the tile's edge rows); tiled kernel: NT stores off / on
-  const std::vector<int> modes = c->rowk ? std::vector<int>{1, 3, 7, 15} : std::vector<int>{0, 1};
+  // (a plan with mode 0 keeps it: back-to-back passes from one buffer into the other do not show what a state that stays
+  // in the cache gains)
+  const std::vector<int> modes = !c->rowk ? std::vector<int>{0, 1} : c->rplan.MM == 0 ? std::vector<int>{0}
+                                                                                       : std::vector<int>{1, 3, 7, 15};
   for (int nt : modes) {
     if (rc != CLMI_OK) break;
-    for (int xc : {4, 8, 16, 32, 64}) {
+    for (int xc : {4, 8, 16, 24, 32, 64}) {
       TiledPlan p;
       RowsPlan rp;
       if (c->rowk ? !scalar_rows_plan(c->N, c->cfg.n_scalars, c->f32, xc, nt, rows_shape(c->cfg.flags), &rp)

@@ -11,7 +11,8 @@
 // chunk.  Memory mode MM: bit 0 non-temporal stores, bit 1 non-temporal loads of the momenta (read
 // exactly once), bit 2 non-temporal loads of the workgroup's own field rows (the y-halo rows, which
 // the neighbouring tile also reads, always use ordinary loads), bit 3 (with bit 2) ordinary loads for
-// the tile's first and last rows, which are the neighbouring tiles' halo rows.
+// the tile's first and last rows, which are the neighbouring tiles' halo rows.  Mode 0, ordinary accesses throughout,
+// is for states that stay in the last-level cache (default_mem_mode).
 //
 // Volume sums are written per (group of G planes, TY-row y-tile), independent of XC.
 #pragma once

@@ -17,22 +17,31 @@ hipError_t launch_scalar_rows_f64_nf2(bool drift, bool kick, bool red, const Sca
     case 15: return dispatch_rows<NF_, false, VZ_, WPR_, TY_, 15, PK_>(drift, kick, red, a, p.blocks, p.XC, p.G, s, kick2); \
     default: return hipErrorInvalidValue;                                                              \
   }
+// memory mode 0 (64^3 to 192^3 only)
+#define CLMI_MM0(NF_, VZ_, PK_)                                                                          \
+  if (p.MM == 0)                                                                                       \
+    return dispatch_rows<NF_, false, VZ_, 1, 8, 0, PK_>(drift, kick, red, a, p.blocks, p.XC, p.G, s, kick2);
 #define CLMI_SHAPE(NF_, VZ_, WPR_, TY_)                                                                  \
   if (p.VZ == VZ_ && p.WPR == WPR_ && p.TY == TY_) CLMI_MM(NF_, VZ_, WPR_, TY_, 0)
-#define CLMI_SHAPE_PK(NF_, VZ_, WPR_, TY_)                                                               \
-  if (p.VZ == VZ_ && p.WPR == WPR_ && p.TY == TY_) {                                                   \
-    if (pk == 1) CLMI_MM(NF_, VZ_, WPR_, TY_, 1)                                                        \
-    CLMI_MM(NF_, VZ_, WPR_, TY_, 0)                                                                     \
+#define CLMI_SHAPE_PK0(NF_, VZ_)                                                                         \
+  if (p.VZ == VZ_ && p.WPR == 1 && p.TY == 8) {                                                        \
+    if (pk == 1) {                                                                                     \
+      CLMI_MM0(NF_, VZ_, 1)                                                                            \
+      CLMI_MM(NF_, VZ_, 1, 8, 1)                                                                       \
+    }                                                                                                  \
+    CLMI_MM0(NF_, VZ_, 0)                                                                              \
+    CLMI_MM(NF_, VZ_, 1, 8, 0)                                                                         \
   }
   CLMI_SHAPE(2, 2, 2, 8)
   CLMI_SHAPE(2, 4, 1, 8)
-  CLMI_SHAPE_PK(2, 2, 1, 8)
-  CLMI_SHAPE_PK(2, 1, 1, 8)
-  CLMI_SHAPE_PK(2, 3, 1, 8)
+  CLMI_SHAPE_PK0(2, 2)
+  CLMI_SHAPE_PK0(2, 1)
+  CLMI_SHAPE_PK0(2, 3)
   CLMI_SHAPE(2, 2, 4, 4)
   CLMI_SHAPE(2, 2, 2, 4)
   CLMI_SHAPE(2, 4, 1, 4)
-#undef CLMI_SHAPE_PK
+#undef CLMI_SHAPE_PK0
+#undef CLMI_MM0
 #undef CLMI_MM
 #undef CLMI_SHAPE
   return hipErrorInvalidValue;

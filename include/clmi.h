@@ -53,11 +53,12 @@ extern "C" {
  * instead of 4-row tiles.  Fields bit-identical; volume sums differ in summation order only. */
 #define CLMI_FLAG_GAUGE_TY8 16
 /* clmi_config.flags: run velocity Verlet as two passes per stage.  By default, for scalar-singlet
- * models on the full-row or tiled lattice pass, the second half-kick of each stage and the first half-kick of
+ * models on the full-row, tiled or plane-chunk lattice pass, the second half-kick of each stage and the first half-kick of
  * the next run in one pass (they read the same fields with the same coefficients); the results are
- * bit-identical either way.  The flag exists for testing. */
+ * bit-identical either way.  It also turns the resident evolver off.  The flag exists for testing. */
 #define CLMI_FLAG_NO_DOUBLE_KICK 32
-/* clmi_config.flags: memory mode m of the full-row lattice pass (0 = the library's default, 15; 1 =
+/* clmi_config.flags: memory mode m of the full-row lattice pass (0 = the library's default: ordinary
+ * accesses where both buffers of the state fit the 256 MB last-level cache (64^3 to 192^3), else 1; 1 =
  * non-temporal stores, 3 = also non-temporal loads of the momenta, 7 = also of the workgroup's own
  * field rows, 15 = as 7 but ordinary loads for the tile's first and last rows).  Results do not
  * depend on it; clmi_autotune chooses one.  This flag, like the shape flags, also selects the
