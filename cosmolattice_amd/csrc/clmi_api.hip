@@ -144,7 +144,8 @@ size_t bytes_field(bool f32) { return f32 ? 4 : 8; }
 // FP64 (134 MB) 27.8 / 32.5 / 33.9, 192^3 one field FP64 (226 MB) 43.5 / 56 / 61; past the cache 192^3 two fields
 // FP32-bulk (340 MB) 86.5 / 82.7 / 84.4 and FP64 (453 MB) 124 / 112 / 123, 256^3 FP32-bulk 181 / 177 / 174, 512^3 - / 1457 /
 // 1510 to 1700.
-int default_mem_mode(double bytes) { return bytes <= 256.0 * 1048576.0 ? 0 : 1; }
+constexpr double kCacheBytes = 256.0 * 1048576.0;
+int default_mem_mode(double bytes) { return bytes <= kCacheBytes ? 0 : 1; }
 
 int rows_shape(int flags)
 {
@@ -182,6 +183,7 @@ double fused_pass_bytes(const clmi_ctx *c)
   if (c->cfg.n_u1 > 0) per_site += 3 * 2.0 * (bf + bp);
   return per_site * (double)c->V;
 }
+bool stays_cached(const clmi_ctx *c) { return fused_pass_bytes(c) <= kCacheBytes; }
 
 int prof_flush(clmi_ctx *c)
 {
@@ -418,7 +420,7 @@ int run_pass(clmi_ctx *c, bool drift, bool kick, bool red, double cdt_s, double 
     if (red && (size_t)r + c->rows_g > c->partial_rows)
       return fail(c, CLMI_E_INVALID, "partial-sum buffer too small for the charged-scalar pass");
     if (c->gtiled)
-      HIPCHK(c, launch_gauge_tiled(c->f32, c->gTY, drift, kick, red, a, c->blocks_g, c->gXC, c->stream));
+      HIPCHK(c, launch_gauge_tiled(c->f32, c->gTY, drift, kick, red, a, c->blocks_g, c->gXC, stays_cached(c), c->stream));
     else
       HIPCHK(c, launch_gauge_pass(c->f32, drift, kick, red, a, c->blocks_g, c->stream));
     if (red) r += c->rows_g;
@@ -2272,7 +2274,7 @@ int autotune_gauge(clmi_ctx *c, int reps, std::string &rep)
   for (int xc = 4; xc <= c->N && e == hipSuccess; xc *= 2) {
     int blocks = 0, rows = 0;
     if (!gauge_tiled_shape(c->N, c->gTY, xc, &blocks, &rows) || rows != c->rows_g) continue;
-    auto launch = [&]() { return launch_gauge_tiled(c->f32, c->gTY, true, true, true, a, blocks, xc, c->stream); };
+    auto launch = [&]() { return launch_gauge_tiled(c->f32, c->gTY, true, true, true, a, blocks, xc, stays_cached(c), c->stream); };
     e = launch();
     if (e == hipSuccess) e = hipEventRecord(e0, c->stream);
     for (int i = 0; i < reps && e == hipSuccess; ++i) e = launch();

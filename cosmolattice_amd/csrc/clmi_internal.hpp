@@ -232,7 +232,7 @@ __device__ __forceinline__ void block_reduce_store(double (&v)[K], double *row)
 bool gauge_tiled_shape(int N, int ty, int XC, int *blocks, int *rows);
 bool gauge_tiled_plan(int N, int ty, int ncu, int *XC, int *blocks, int *rows);
 hipError_t launch_gauge_tiled(bool f32, int ty, bool drift, bool kick, bool red, const GaugePassArgs &a, int blocks,
-                              int XC, hipStream_t s);
+                              int XC, bool plain, hipStream_t s);
 
 // ---- ensembles: several lattices in one launch (scalar_rows_batch.hip, background.hip) ----
 struct RowsMember {   // one lattice's fused pass inside a batched launch (device-resident table)

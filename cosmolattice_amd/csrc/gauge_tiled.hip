@@ -108,7 +108,7 @@ template <bool F32, bool NT> __device__ __forceinline__ void store_v(void *f, fl
 // U1: the lattice has a U(1) field, known at compile time (1) or read from the arguments (0).  Fixing it
 // removes the per-site selects and branches on it; that pays for FP32-bulk (256^3 pass 479 -> 462 us)
 // and not for FP64 (670 -> 683 us), so only FP32-bulk lattices with a U(1) field use U1 = 1.
-template <bool F32, bool DRIFT, bool KICK, bool RED, int GTY, int U1 = 0, bool RAG = false>
+template <bool F32, bool DRIFT, bool KICK, bool RED, int GTY, int U1 = 0, bool RAG = false, bool NT = !RAG>
 __global__ __launch_bounds__(64 * GTY) void k_gauge_tiled(const GaugePassArgs a, const int XC, const int RG)
 {
   using G = GVal<F32>;
@@ -239,9 +239,9 @@ __global__ __launch_bounds__(64 * GTY) void k_gauge_tiled(const GaugePassArgs a,
 
     const uint32_t s = site(x, y, z);
     if (DRIFT && act) {
-      for (int q = 0; q < 2; ++q) store_v<F32, !RAG>(a.phi_out[q], a.philo_out[q], s, g.fc[q]);
+      for (int q = 0; q < 2; ++q) store_v<F32, NT>(a.phi_out[q], a.philo_out[q], s, g.fc[q]);
       if (u1)
-        for (int d = 0; d < 3; ++d) store_v<F32, !RAG>(a.A_out[d], a.Alo_out[d], s, g.Ac[d]);
+        for (int d = 0; d < 3; ++d) store_v<F32, NT>(a.A_out[d], a.Alo_out[d], s, g.Ac[d]);
     }
     P pin[2], pAin[3] = {0, 0, 0}, pout[2], pAout[3];
     if (KICK) {
@@ -258,9 +258,9 @@ __global__ __launch_bounds__(64 * GTY) void k_gauge_tiled(const GaugePassArgs a,
     else
       gauge_site_f64<KICK, RED>(k, a.poly, g, pin, pAin, pout, pAout, acc);
     if (KICK && act) {
-      for (int q = 0; q < 2; ++q) store_out<!RAG>((P *)a.pi_out[q] + s, pout[q]);
+      for (int q = 0; q < 2; ++q) store_out<NT>((P *)a.pi_out[q] + s, pout[q]);
       if (u1)
-        for (int d = 0; d < 3; ++d) store_out<!RAG>((P *)a.piA_out[d] + s, pAout[d]);
+        for (int d = 0; d < 3; ++d) store_out<NT>((P *)a.piA_out[d] + s, pAout[d]);
     }
     if (RED && ((x + 1) % RG == 0 || (RAG && x + 1 == N))) {
       double v[kNumRed] = {0, 0, acc[2], acc[0], acc[1], acc[3], acc[4], 0};
@@ -283,14 +283,14 @@ __global__ __launch_bounds__(64 * GTY) void k_gauge_tiled(const GaugePassArgs a,
   }
 }
 
-template <bool F32, int GTY, int U1 = 0, bool RAG = false>
+template <bool F32, int GTY, int U1 = 0, bool RAG = false, bool NT = !RAG>
 hipError_t dispatch_tiled(bool drift, bool kick, bool red, const GaugePassArgs &a, int blocks, int XC, hipStream_t s)
 {
   const int G = gauge_rows_g((int)a.N);
   const int code = (drift ? 4 : 0) | (kick ? 2 : 0) | (red ? 1 : 0);
 #define CLMI_GT(D, K, R)                                                                                  \
   case ((D ? 4 : 0) | (K ? 2 : 0) | (R ? 1 : 0)):                                                        \
-    hipLaunchKernelGGL((k_gauge_tiled<F32, D, K, R, GTY, U1, RAG>), dim3(blocks), dim3(64 * GTY), 0, s, a, XC, G); \
+    hipLaunchKernelGGL((k_gauge_tiled<F32, D, K, R, GTY, U1, RAG, NT>), dim3(blocks), dim3(64 * GTY), 0, s, a, XC, G); \
     break;
   switch (code) {
     CLMI_GT(true, true, true)
@@ -359,8 +359,11 @@ bool gauge_tiled_plan(int N, int ty, int ncu, int *XC, int *blocks, int *rows)
   return gauge_tiled_shape(N, ty, best, blocks, rows);
 }
 
+// plain (the state stays in the last-level cache): ordinary stores, so that the next pass reads it from there; else
+// non-temporal ones.  Only FP32-bulk lattices gain: 128^3 (252 MB in both buffers), a leapfrog step 75 -> 60.5 us, while 64^3
+// is the same either way and FP64 at 128^3 (335 MB) 96 -> 100.
 hipError_t launch_gauge_tiled(bool f32, int ty, bool drift, bool kick, bool red, const GaugePassArgs &a, int blocks,
-                              int XC, hipStream_t s)
+                              int XC, bool plain, hipStream_t s)
 {
   const bool u1 = a.has_u1 != 0;
   if (a.N % GTZ != 0)
@@ -371,6 +374,8 @@ hipError_t launch_gauge_tiled(bool f32, int ty, bool drift, bool kick, bool red,
     return f32 ? (u1 ? dispatch_tiled<true, 8, 1>(drift, kick, red, a, blocks, XC, s)
                      : dispatch_tiled<true, 8>(drift, kick, red, a, blocks, XC, s))
                : dispatch_tiled<false, 8>(drift, kick, red, a, blocks, XC, s);
+  if (ty == 4 && f32 && u1 && plain)
+    return dispatch_tiled<true, 4, 1, false, false>(drift, kick, red, a, blocks, XC, s);
   if (ty == 4)
     return f32 ? (u1 ? dispatch_tiled<true, 4, 1>(drift, kick, red, a, blocks, XC, s)
                      : dispatch_tiled<true, 4>(drift, kick, red, a, blocks, XC, s))
