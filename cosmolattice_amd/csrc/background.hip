@@ -96,23 +96,53 @@ __global__ __launch_bounds__(kBlock) void k_gauss(const GaussArgs a)
 template <bool F32>
 __global__ __launch_bounds__(kBlock) void k_means(const MeansArgs a)
 {
+  // A thread takes two z-neighbours (N is even) at a time and U pairs per turn, every load of them in flight: a load a
+  // site and turn, with a division for its coordinates, ran at 2.7 TB/s (256^3 FP64 with the gradient 50 -> 35 us).
+  constexpr int U = 2;
   double acc[3] = {0, 0, 0};
+  struct Two {
+    double a, b;
+  };
+  auto ld2 = [&](uint32_t i) -> Two {
+    if constexpr (F32) {
+      const float2 h = *(const float2 *)((const float *)a.p + i);
+      const float2 l = a.lo ? *(const float2 *)(a.lo + i) : float2{0.0f, 0.0f};
+      return {(double)h.x + (double)l.x, (double)h.y + (double)l.y};
+    } else {
+      const double2 h = *(const double2 *)((const double *)a.p + i);
+      return {h.x, h.y};
+    }
+  };
   auto ld = [&](uint32_t i) -> double {
     if (F32) return (double)((const float *)a.p)[i] + (a.lo ? (double)a.lo[i] : 0.0);
     return ((const double *)a.p)[i];
   };
-  const uint32_t N = a.N, NN = N * N;
-  for (uint32_t s = blockIdx.x * kBlock + threadIdx.x; s < a.V; s += gridDim.x * kBlock) {
-    const double c = ld(s);
-    const double v = c * a.scale;
-    acc[0] += v;
-    acc[1] += v * v;
-    if (a.grad) {
-      const uint32_t x = s / NN, y = (s - x * NN) / N, z = s - x * NN - y * N;
-      const double dx = ld(s - x * NN + (x + 1 == N ? 0 : x + 1) * NN) - c;
-      const double dy = ld(s - y * N + (y + 1 == N ? 0 : y + 1) * N) - c;
-      const double dz = ld(s - z + (z + 1 == N ? 0 : z + 1)) - c;
-      acc[2] += dx * dx + dy * dy + dz * dz;
+  const uint32_t N = a.N, NN = N * N, pairs = a.V / 2, stride = gridDim.x * kBlock;
+  for (uint32_t i = blockIdx.x * kBlock + threadIdx.x; i < pairs; i += U * stride) {
+    Two c[U], nx[U], ny[U];
+    double nz[U];
+#pragma unroll
+    for (int u = 0; u < U; ++u) {
+      const uint32_t s = 2 * (i + u * stride < pairs ? i + u * stride : i);
+      c[u] = ld2(s);
+      if (a.grad) {
+        const uint32_t x = s / NN, y = (s - x * NN) / N, z = s - x * NN - y * N;
+        nx[u] = ld2(s - x * NN + (x + 1 == N ? 0 : x + 1) * NN);
+        ny[u] = ld2(s - y * N + (y + 1 == N ? 0 : y + 1) * N);
+        nz[u] = ld(z + 2 == N ? s - z : s + 2);
+      }
+    }
+#pragma unroll
+    for (int u = 0; u < U; ++u) {
+      if (i + u * stride >= pairs) break;
+      const double v0 = c[u].a * a.scale, v1 = c[u].b * a.scale;
+      acc[0] += v0 + v1;
+      acc[1] += v0 * v0 + v1 * v1;
+      if (a.grad) {
+        const double xa = nx[u].a - c[u].a, xb = nx[u].b - c[u].b, ya = ny[u].a - c[u].a, yb = ny[u].b - c[u].b;
+        const double za = c[u].b - c[u].a, zb = nz[u] - c[u].b;
+        acc[2] += (xa * xa + ya * ya + za * za) + (xb * xb + yb * yb + zb * zb);
+      }
     }
   }
   double v[kNumRed] = {acc[0], acc[1], acc[2], 0, 0, 0, 0, 0};

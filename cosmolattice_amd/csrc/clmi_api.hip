@@ -88,8 +88,8 @@ struct clmi_ctx {
   double *stage = nullptr;  // N^3 doubles
   void *fk = nullptr;       // N*N*(N/2+1) double2
   void *fk2 = nullptr;
-  hipfftHandle plan_r2c = 0, plan_c2r = 0;
-  bool have_r2c = false, have_c2r = false;
+  hipfftHandle plan_r2c = 0, plan_c2r = 0, plan_yz = 0;  // plan_yz: real to complex over y and z, every x plane
+  bool have_r2c = false, have_c2r = false, have_yz = false;
   BinTable bins;
   double *bin_out = nullptr;
   int bin_out_n = 0;
@@ -590,7 +590,7 @@ int ensure_stage(clmi_ctx *c)
   return CLMI_OK;
 }
 
-int ensure_fft(clmi_ctx *c, bool r2c, bool c2r, bool two)
+int ensure_fft(clmi_ctx *c, bool r2c, bool c2r, bool two, bool planes = false)
 {
   CHK(ensure_stage(c));
   const size_t nm = (size_t)c->N * c->N * (c->N / 2 + 1);
@@ -600,6 +600,12 @@ int ensure_fft(clmi_ctx *c, bool r2c, bool c2r, bool two)
     FFTCHK(c, hipfftPlan3d(&c->plan_r2c, c->N, c->N, c->N, HIPFFT_D2Z));
     FFTCHK(c, hipfftSetStream(c->plan_r2c, c->stream));
     c->have_r2c = true;
+  }
+  if (planes && !c->have_yz) {
+    int n[2] = {c->N, c->N};
+    FFTCHK(c, hipfftPlanMany(&c->plan_yz, 2, n, nullptr, 1, 0, nullptr, 1, 0, HIPFFT_D2Z, c->N));
+    FFTCHK(c, hipfftSetStream(c->plan_yz, c->stream));
+    c->have_yz = true;
   }
   if (c2r && !c->have_c2r) {
     FFTCHK(c, hipfftPlan3d(&c->plan_c2r, c->N, c->N, c->N, HIPFFT_Z2D));
@@ -834,6 +840,7 @@ void clmi_destroy(clmi_ctx *c)
   if (c->bin_out) (void)hipFree(c->bin_out);
   free_bin_table(c->bins);
   if (c->have_r2c) (void)hipfftDestroy(c->plan_r2c);
+  if (c->have_yz) (void)hipfftDestroy(c->plan_yz);
   if (c->have_c2r) (void)hipfftDestroy(c->plan_c2r);
   for (hipEvent_t e : c->ev) (void)hipEventDestroy(e);
   if (c->bounce) (void)hipHostFree(c->bounce);
@@ -1338,19 +1345,24 @@ int clmi_spectrum_bins_npow(clmi_ctx *c, int kind, int index, int comp, double d
     return fail(c, CLMI_E_INVALID, "nbins must equal clmi_spectrum_nbins(ctx, dk)");
   if (npow != 0 && npow != 1 && npow != 3) return fail(c, CLMI_E_INVALID, "npow must be 0, 1 or 3");
   CHK(flush(c));
+  if (c->bins.nbins != nbins || c->bins.dk != dk || c->bins.N != c->N) {
+    CHK(sync_stream(c));
+    HIPCHK(c, build_bin_table(c->bins, c->N, dk, nbins));
+  }
+  const bool xdft = c->bins.d_tw != nullptr;  // the x transform runs with the binning
   double *fft_in = nullptr;
   if (kind == CLMI_MAG_U1) {
     if (comp < 0 || comp > 2) return fail(c, CLMI_E_INVALID, "CLMI_MAG_U1: comp must be 0, 1 or 2");
     NormArgs a{};
     CHK(u1_curl_args(c, index, &a));
-    CHK(ensure_fft(c, true, false, false));
+    CHK(ensure_fft(c, !xdft, false, false, xdft));
     HIPCHK(c, launch_curl_component(a, comp, c->stage, c->stream));
     fft_in = c->stage;
   } else {
     DevArr *arr = nullptr;
     bool is_field = false;
     CHK(select_arr(c, kind, index, comp, &arr, &is_field));
-    CHK(ensure_fft(c, true, false, false));
+    CHK(ensure_fft(c, !xdft, false, false, xdft));
     if (c->f32) {
       HIPCHK(c, launch_join_f64((const float *)arr->p, arr->lo, c->stage, c->V, c->stream));
       fft_in = c->stage;
@@ -1358,11 +1370,7 @@ int clmi_spectrum_bins_npow(clmi_ctx *c, int kind, int index, int comp, double d
       fft_in = (double *)arr->p;  // the out-of-place R2C transform reads the array and leaves it unchanged
     }
   }
-  FFTCHK(c, hipfftExecD2Z(c->plan_r2c, (hipfftDoubleReal *)fft_in, (hipfftDoubleComplex *)c->fk));
-  if (c->bins.nbins != nbins || c->bins.dk != dk || c->bins.N != c->N) {
-    CHK(sync_stream(c));
-    HIPCHK(c, build_bin_table(c->bins, c->N, dk, nbins));
-  }
+  FFTCHK(c, hipfftExecD2Z(xdft ? c->plan_yz : c->plan_r2c, (hipfftDoubleReal *)fft_in, (hipfftDoubleComplex *)c->fk));
   if (c->bin_out_n < nbins) {
     if (c->bin_out) HIPCHK(c, hipFree(c->bin_out));
     c->bin_out = nullptr;
@@ -1370,7 +1378,8 @@ int clmi_spectrum_bins_npow(clmi_ctx *c, int kind, int index, int comp, double d
     HIPCHK(c, hipMalloc(&c->bin_out, sizeof(double) * nbins));
     c->bin_out_n = nbins;
   }
-  HIPCHK(c, launch_bin_sums(c->bins, c->fk, c->bin_out, c->stream, npow));
+  HIPCHK(c, xdft ? launch_xdft_bins(c->bins, c->fk, c->bin_out, c->stream, npow)
+                 : launch_bin_sums(c->bins, c->fk, c->bin_out, c->stream, npow));
   HIPCHK(c, hipMemcpyAsync(sum_f2, c->bin_out, sizeof(double) * nbins, hipMemcpyDeviceToHost, c->stream));
   CHK(sync_stream(c));
   for (int b = 0; b < nbins; ++b) {

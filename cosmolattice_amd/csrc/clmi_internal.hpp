@@ -501,6 +501,10 @@ struct BinTable {
   // bin-sorted index table (more bins)
   uint32_t *d_modes = nullptr;   // half-space mode indices sorted by bin
   uint32_t *d_start = nullptr;   // nbins + 1 offsets
+  // fused x transform (xdft_length(N)): its twiddles W_N^k (double2), workgroups, column blocks each
+  double *d_tw = nullptr;
+  int xgroups = 0;
+  uint32_t xper = 0;
   std::vector<double> count, mean_n;
 };
 hipError_t build_bin_table(BinTable &t, int N, double dk, int nbins);
@@ -508,6 +512,10 @@ void free_bin_table(BinTable &t);
 // out[b] = sum over the modes of bin b of w |f_k|^2 |n|^npow (npow = 0, 1 or 3; w = 2 for the modes the
 // R2C half-space stands for twice).
 hipError_t launch_bin_sums(const BinTable &t, const void *fk /*double2*/, double *out, hipStream_t s, int npow = 0);
+// The same from fk transformed over y and z only: the x transform and the sums in one pass, where the table has
+// twiddles (d_tw; powers of two 64 to 256, whose lines fit a thread's registers twice over).
+bool xdft_length(int N);
+hipError_t launch_xdft_bins(const BinTable &t, const void *fk, double *out, hipStream_t s, int npow);
 
 struct GrfArgs {
   int N;
