@@ -362,18 +362,27 @@ GaugePassArgs gauge_args(const clmi_ctx *c, int fi, int fo, int pi, int po, doub
   return a;
 }
 
+// Whether velocity-Verlet stages may share a double-kick pass: scalar singlets alone, on the full-row, the tiled or the
+// plane-chunk pass; a charged scalar (with or without U(1)) alone, on its tiled pass with 4-row tiles.
+bool double_kick_ok(const clmi_ctx *c)
+{
+  if (c->cfg.flags & CLMI_FLAG_NO_DOUBLE_KICK) return false;
+  if (c->cfg.n_cscalars == 0) return (c->rowk || c->tiled || c->flat) && c->cfg.n_scalars > 0;
+  return c->cfg.n_scalars == 0 && c->gtiled && c->gTY == 4;
+}
+
 // Launch one lattice pass over every sector; returns the number of partial rows written in *rows.
 // ops (reducing passes): run this background update in the pass's last workgroup; *updated says whether it does.  The
 // scalar-singlet full-row and plane-chunk passes do (what it gains: pass_tail.hpp), but for a pass that is timed by
 // itself and a model whose update needs the general power.
-// ckick2_s != 0 (drift + kick passes of scalar-singlet models on the full-row pass): kick the scalars a
-// second time, by ckick2_s, from the same drifted fields (see double_kick_ok).
+// ckick2_s, ckick2_g != 0 (drift + kick passes, see double_kick_ok): kick a second time, the scalars by ckick2_s, the
+// charged scalar and U(1) by ckick2_g, from the same drifted fields.
 int run_pass(clmi_ctx *c, bool drift, bool kick, bool red, double cdt_s, double ckick_s, double ckick_g, int *rows,
-             double ckick2_s = 0.0, const UpdateOps *ops = nullptr, bool *updated = nullptr)
+             double ckick2_s = 0.0, double ckick2_g = 0.0, const UpdateOps *ops = nullptr, bool *updated = nullptr)
 {
   const bool kick2 = ckick2_s != 0.0;
-  if (kick2 && !(drift && kick && (c->rowk || c->tiled || c->flat) && c->cfg.n_cscalars == 0))
-    return fail(c, CLMI_E_INVALID, "double kick outside a scalar-singlet full-row, tiled or plane-chunk drift + kick pass");
+  if (kick2 && !(drift && kick && double_kick_ok(c)))
+    return fail(c, CLMI_E_INVALID, "double kick outside a drift + kick pass that has one");
   const bool timed = c->prof && drift && kick && (c->prof_count++ % c->prof_every == 0);
   if (timed) CHK(prof_event(c));
   PassTail tail{};
@@ -416,7 +425,8 @@ int run_pass(clmi_ctx *c, bool drift, bool kick, bool red, double cdt_s, double 
   if (c->cfg.n_cscalars > 0) {
     const int fi = c->cur_fG, fo = drift ? 1 - c->cur_fG : c->cur_fG;
     const int pi = c->cur_pG, po = (drift && kick) ? 1 - c->cur_pG : c->cur_pG;
-    const GaugePassArgs a = gauge_args(c, fi, fo, pi, po, cdt_s, ckick_g, r);
+    GaugePassArgs a = gauge_args(c, fi, fo, pi, po, cdt_s, ckick_g, r);
+    a.ckick2 = ckick2_g;
     if (red && (size_t)r + c->rows_g > c->partial_rows)
       return fail(c, CLMI_E_INVALID, "partial-sum buffer too small for the charged-scalar pass");
     if (c->gtiled)
@@ -453,7 +463,7 @@ int update(clmi_ctx *c, int rows, std::initializer_list<std::pair<int, double>> 
 // context holds a snapshot target (c->snap) and the update starts with storeFieldsAverages, the
 // background after that operation -- the state a flush at this point would leave -- is written there.
 int pass_update(clmi_ctx *c, bool drift, bool kick, bool red, double cdt_s, double ckick_s, double ckick_g,
-                bool do_update, std::initializer_list<std::pair<int, double>> ops, double ckick2_s = 0.0)
+                bool do_update, std::initializer_list<std::pair<int, double>> ops, double ckick2_s = 0.0, double ckick2_g = 0.0)
 {
   int rows = 0;
   bool updated = false;
@@ -462,16 +472,9 @@ int pass_update(clmi_ctx *c, bool drift, bool kick, bool red, double cdt_s, doub
     u.snap = c->snap;
     c->snap = nullptr;
   }
-  CHK(run_pass(c, drift, kick, red, cdt_s, ckick_s, ckick_g, &rows, ckick2_s, do_update ? &u : nullptr, &updated));
+  CHK(run_pass(c, drift, kick, red, cdt_s, ckick_s, ckick_g, &rows, ckick2_s, ckick2_g, do_update ? &u : nullptr, &updated));
   if (do_update && !updated) HIPCHK(c, launch_update(c->dstate, c->partials, rows, c->mc, u, c->stream));
   return CLMI_OK;
-}
-
-// Whether velocity-Verlet stages may share a double-kick pass: scalar singlets only, on the full-row, the
-// tiled or the plane-chunk pass.
-bool double_kick_ok(const clmi_ctx *c)
-{
-  return (c->rowk || c->tiled || c->flat) && c->cfg.n_scalars > 0 && c->cfg.n_cscalars == 0 && !(c->cfg.flags & CLMI_FLAG_NO_DOUBLE_KICK);
 }
 
 // Fewest passes that the resident evolver takes: a cooperative launch with its load and store of the state costs
@@ -983,7 +986,8 @@ int clmi_vv_evolve(clmi_ctx *c, const double *ws, int nws, int nsteps)
   const double dt = c->cfg.dt;
   const int stages = (nws - 1) * 2 + 1;
   auto weight = [&](int s) { return ws[s < nws ? s : stages - s - 1]; };
-  if (double_kick_ok(c)) {
+  // (a kick of weight zero is no second kick to a pass)
+  if (double_kick_ok(c) && std::all_of(ws, ws + nws, [&](double w) { return w * dt / 2 != 0.0 && dt / 2 * w != 0.0; })) {
     // The second half-kick of a stage and the first half-kick of the next read the same drifted fields,
     // and the scale-factor operations between them change aDot but not a_I, so both kicks have the
     // same coefficients: one double-kick pass gives exactly the momenta, and in its two sums exactly
@@ -1004,7 +1008,7 @@ int clmi_vv_evolve(clmi_ctx *c, const double *ws, int nws, int nsteps)
         CHK(pass_update(c, true, true, ex, dt * w, w * dt / 2, dt / 2 * w, ex,
                         {{OP_STORE_FIELDS, 0.0}, {OP_VV_MOMENTA, 0.0}, {OP_VV_SF_ONE, w}, {OP_VV_SF_HALF, w2},
                          {OP_VV_MOMENTA_KICK2, 0.0}, {OP_VV_DRIFT_SF, w2}},
-                        w2 * dt / 2));
+                        w2 * dt / 2, dt / 2 * w2));
       } else {
         CHK(pass_update(c, true, true, ex, dt * w, w * dt / 2, dt / 2 * w, ex,
                         {{OP_STORE_FIELDS, 0.0}, {OP_VV_MOMENTA, 0.0}, {OP_VV_SF_ONE, w}}));

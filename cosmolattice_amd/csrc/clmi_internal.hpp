@@ -31,6 +31,9 @@ enum RedSlot : int {
   RED_PI2U1 = 5,
   RED_B2U1 = 6,
   RED_PI2S_KICK2 = 7,  // scalar momenta after the second kick of a double-kick pass
+  // the same of a charged scalar and its U(1) field; such passes run without scalar singlets, whose slots these are
+  RED_PI2CS_KICK2 = 0,
+  RED_PI2U1_KICK2 = 1,
 };
 
 // Device-resident homogeneous state plus the per-pass coefficients derived from it.
@@ -155,6 +158,7 @@ struct GaugePassArgs {
   double jnorm;  // 2/dx * (fStar/omegaStar)^2
   double cdt;
   double ckick;
+  double ckick2;  // of the second kick of a double-kick pass, else 0
   const DevState *st;
   double *partials;
   CsPoly poly;

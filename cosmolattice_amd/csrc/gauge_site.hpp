@@ -36,12 +36,12 @@ struct GaugeIn {
   V Ad[3][3];     // [i][j]: A_j(x + i - j), i != j
 };
 
-// Kick and reduction constants of one pass.
+// Kick and reduction constants of one pass (those ending in 2: of a double-kick pass's second kick).
 struct GaugeK {
   // FP64
-  double ckick, aK, aV, aG, aJ, inv_dx, inv_dx2, dx, gQ, jnorm;
+  double ckick, ckick2, aK, aV, aG, aJ, inv_dx, inv_dx2, dx, gQ, jnorm;
   // FP32-bulk
-  float kK, kV, kG, kJ, th_scale;
+  float kK, kV, kG, kJ, kK2, kV2, kG2, kJ2, th_scale;
   bool u1;
 };
 
@@ -102,10 +102,12 @@ __device__ __forceinline__ void pair_add(float &hi, float &lo, float d)
 }
 
 // FP64 site update.  pin, pAin: momenta at x (read); pout, pAout: kicked momenta; acc: the five sums.
-template <bool KICK, bool RED>
+// KICK2: the momenta are kicked a second time from the same fields; acc[0] and acc[3] hold the sums after the first kick,
+// acc[5] and acc[6] those after the second.
+template <bool KICK, bool RED, bool KICK2 = false>
 __device__ __forceinline__ void gauge_site_f64(const GaugeK &k, const CsPoly &poly, const GaugeIn<double> &g,
                                                const double pin[2], const double pAin[3], double pout[2],
-                                               double pAout[3], double acc[5])
+                                               double pAout[3], double *acc)
 {
   const double pr = g.fc[0], pim = g.fc[1];
   double plus_r = 0, plus_i = 0, minus_r = 0, minus_i = 0, g2 = 0;
@@ -136,22 +138,30 @@ __device__ __forceinline__ void gauge_site_f64(const GaugeK &k, const CsPoly &po
   }
   const double r2 = pr * pr + pim * pim;
   double p_r = pin[0], p_i = pin[1];
+  double p2 = 0.0;  // after the first kick (KICK2)
   if (KICK) {
     const double lap_r = (plus_r + minus_r - 6 * pr) * k.inv_dx2;
     const double lap_i = (plus_i + minus_i - 6 * pim) * k.inv_dx2;
     const double nd = cs_dnorm_over_norm_d(poly, r2);
-    p_r += k.ckick * (k.aK * lap_r - k.aV / 2 * (nd * pr));
-    p_i += k.ckick * (k.aK * lap_i - k.aV / 2 * (nd * pim));
+    const double F_r = k.aK * lap_r - k.aV / 2 * (nd * pr), F_i = k.aK * lap_i - k.aV / 2 * (nd * pim);
+    p_r += k.ckick * F_r;
+    p_i += k.ckick * F_i;
+    if (KICK2) {
+      p2 = p_r * p_r + p_i * p_i;
+      p_r += k.ckick2 * F_r;
+      p_i += k.ckick2 * F_i;
+    }
   }
   pout[0] = p_r;
   pout[1] = p_i;
   if (RED) {
-    acc[0] += p_r * p_r + p_i * p_i;
+    if (KICK2) acc[0] += p2;
+    acc[KICK2 ? 5 : 0] += p_r * p_r + p_i * p_i;
     acc[1] += g2;
     acc[2] += cs_pot_d(poly, r2);
   }
   if (k.u1) {
-    double e2 = 0.0;
+    double e2 = 0.0, e2a = 0.0;  // e2a: after the first kick (KICK2)
     for (int i = 0; i < 3; ++i) {
       double pa = pAin[i];
       if (KICK) {
@@ -169,7 +179,12 @@ __device__ __forceinline__ void gauge_site_f64(const GaugeK &k, const CsPoly &po
         const double ur = cl[i] * fpr - sl[i] * fpi;
         const double ui = cl[i] * fpi + sl[i] * fpr;
         const double J = k.jnorm * k.gQ * (ur * pim - ui * pr);
-        pa += k.ckick * (k.aG * (lap - gd) - k.aJ * J);
+        const double F = k.aG * (lap - gd) - k.aJ * J;
+        pa += k.ckick * F;
+        if (KICK2) {
+          e2a += pa * pa;
+          pa += k.ckick2 * F;
+        }
       }
       pAout[i] = pa;
       e2 += pa * pa;
@@ -181,7 +196,8 @@ __device__ __forceinline__ void gauge_site_f64(const GaugeK &k, const CsPoly &po
           const double f = ((g.Ap[i][j] - g.Ac[j]) - (g.Ap[j][i] - g.Ac[i])) * k.inv_dx;
           b2 += f * f;
         }
-      acc[3] += e2;
+      if (KICK2) acc[3] += e2a;
+      acc[KICK2 ? 6 : 3] += e2;
       acc[4] += b2;
     }
   }
@@ -206,10 +222,10 @@ __device__ __forceinline__ void link_m1(const GaugeK &k, P2 Ad, float &cm1, floa
 
 // FP32-bulk site update (stencil differences on hi and lo separately, kick and per-site energy terms in
 // FP32, accumulated over sites in FP64, as the scalar FP32-bulk pass does).
-template <bool KICK, bool RED>
+template <bool KICK, bool RED, bool KICK2 = false>
 __device__ __forceinline__ void gauge_site_f32(const GaugeK &k, const CsPoly &poly, const GaugeIn<P2> &g,
                                                const float pin[2], const float pAin[3], float pout[2],
-                                               float pAout[3], double acc[5])
+                                               float pAout[3], double *acc)
 {
   const P2 fr = g.fc[0], fi = g.fc[1];
   const float pr = fr.h + fr.l, pim = fi.h + fi.l;
@@ -237,20 +253,27 @@ __device__ __forceinline__ void gauge_site_f32(const GaugeK &k, const CsPoly &po
     if (RED) g2 += dr * dr + di * di;
   }
   float p_r = pin[0], p_i = pin[1];
+  float p2 = 0.0f;  // after the first kick (KICK2)
   if (KICK) {
     const float nd = cs_dnorm_over_norm_f(poly, pr * pr + pim * pim);
     p_r += k.kK * lap_r - k.kV * (nd * pr);
     p_i += k.kK * lap_i - k.kV * (nd * pim);
+    if (KICK2) {
+      p2 = p_r * p_r + p_i * p_i;
+      p_r += k.kK2 * lap_r - k.kV2 * (nd * pr);
+      p_i += k.kK2 * lap_i - k.kV2 * (nd * pim);
+    }
   }
   pout[0] = p_r;
   pout[1] = p_i;
   if (RED) {
-    acc[0] += (double)(p_r * p_r + p_i * p_i);
+    if (KICK2) acc[0] += (double)p2;
+    acc[KICK2 ? 5 : 0] += (double)(p_r * p_r + p_i * p_i);
     acc[1] += (double)g2 * k.inv_dx2;
     acc[2] += (double)cs_pot_f(poly, pr * pr + pim * pim);
   }
   if (k.u1) {
-    float e2 = 0.0f;
+    float e2 = 0.0f, e2a = 0.0f;  // e2a: after the first kick (KICK2)
     for (int i = 0; i < 3; ++i) {
       float pa = pAin[i];
       if (KICK) {
@@ -268,6 +291,10 @@ __device__ __forceinline__ void gauge_site_f32(const GaugeK &k, const CsPoly &po
         const float ui = (cm[i] + 1.0f) * qif + sl[i] * qrf;
         const float J = ur * pim - ui * pr;
         pa += k.kG * (lap - gd) - k.kJ * J;
+        if (KICK2) {
+          e2a += pa * pa;
+          pa += k.kG2 * (lap - gd) - k.kJ2 * J;
+        }
       }
       pAout[i] = pa;
       e2 += pa * pa;
@@ -279,7 +306,8 @@ __device__ __forceinline__ void gauge_site_f32(const GaugeK &k, const CsPoly &po
           const float f = p2diff(g.Ap[i][j], g.Ac[j]) - p2diff(g.Ap[j][i], g.Ac[i]);
           b2 += f * f;
         }
-      acc[3] += (double)e2;
+      if (KICK2) acc[3] += (double)e2a;
+      acc[KICK2 ? 6 : 3] += (double)e2;
       acc[4] += (double)b2 * k.inv_dx2;
     }
   }
@@ -321,6 +349,7 @@ __device__ __forceinline__ GaugeK gauge_consts(const GaugePassArgs &a, bool kick
 {
   GaugeK k;
   k.ckick = a.ckick;
+  k.ckick2 = a.ckick2;
   k.aK = kick ? a.st->aK : 0.0;
   k.aV = kick ? a.st->aV : 0.0;
   k.aG = kick ? a.st->aG : 0.0;
@@ -334,6 +363,10 @@ __device__ __forceinline__ GaugeK gauge_consts(const GaugePassArgs &a, bool kick
   k.kV = kick ? (float)(a.ckick * a.st->aV * 0.5) : 0.0f;
   k.kG = kick ? (float)(a.ckick * a.st->aG * a.inv_dx2) : 0.0f;
   k.kJ = kick ? (float)(a.ckick * a.st->aJ * a.jnorm * a.gQ) : 0.0f;
+  k.kK2 = kick ? (float)(a.ckick2 * a.st->aK * a.inv_dx2) : 0.0f;
+  k.kV2 = kick ? (float)(a.ckick2 * a.st->aV * 0.5) : 0.0f;
+  k.kG2 = kick ? (float)(a.ckick2 * a.st->aG * a.inv_dx2) : 0.0f;
+  k.kJ2 = kick ? (float)(a.ckick2 * a.st->aJ * a.jnorm * a.gQ) : 0.0f;
   k.th_scale = (float)(-a.dx * a.gQ);
   k.u1 = a.has_u1 != 0;
   return k;

@@ -108,8 +108,15 @@ template <bool F32, bool NT> __device__ __forceinline__ void store_v(void *f, fl
 // U1: the lattice has a U(1) field, known at compile time (1) or read from the arguments (0).  Fixing it
 // removes the per-site selects and branches on it; that pays for FP32-bulk (256^3 pass 479 -> 462 us)
 // and not for FP64 (670 -> 683 us), so only FP32-bulk lattices with a U(1) field use U1 = 1.
-template <bool F32, bool DRIFT, bool KICK, bool RED, int GTY, int U1 = 0, bool RAG = false, bool NT = !RAG>
-__global__ __launch_bounds__(64 * GTY) void k_gauge_tiled(const GaugePassArgs a, const int XC, const int RG)
+//
+// KICK2 (drift + kick passes of velocity Verlet): the closing half-kick of a stage and the opening one of the next read the
+// same fields, so one pass does both and keeps the sums after each.  It is the drift + kick pass plus a few operations,
+// where the second pass moved the whole state again.  A velocity-Verlet step, two passes / one (us, FP64 and FP32-bulk):
+// 64^3 51.1 / 30.5 and 44.8 / 25.6, 100^3 138 / 83 and 112 / 63, 128^3 182 / 120 and 116 / 63, 200^3 815 / 539 and
+// 657 / 399, 256^3 1252 / 862 and 853 / 484.  FP64 asks for two waves a SIMD: left alone it takes two registers more
+// than they have.
+template <bool F32, bool DRIFT, bool KICK, bool RED, int GTY, int U1 = 0, bool RAG = false, bool NT = !RAG, bool KICK2 = false>
+__global__ __launch_bounds__(64 * GTY, KICK2 && !F32 ? 2 : 1) void k_gauge_tiled(const GaugePassArgs a, const int XC, const int RG)
 {
   using G = GVal<F32>;
   using V = typename G::V;
@@ -195,7 +202,7 @@ __global__ __launch_bounds__(64 * GTY) void k_gauge_tiled(const GaugePassArgs a,
   }
   __syncthreads();
 
-  double acc[5] = {0, 0, 0, 0, 0};
+  double acc[7] = {0, 0, 0, 0, 0, 0, 0};
   const int ly = y - y0 + 1, lz = z - z0 + 1;
   for (int x = x0; x < xe; ++x) {
     const bool more = x + 1 < xe;
@@ -254,21 +261,21 @@ __global__ __launch_bounds__(64 * GTY) void k_gauge_tiled(const GaugePassArgs a,
         for (int d = 0; d < 3; ++d) pAin[d] = ((const P *)a.piA_in[d])[s];
     }
     if constexpr (F32)
-      gauge_site_f32<KICK, RED>(k, a.poly, g, pin, pAin, pout, pAout, acc);
+      gauge_site_f32<KICK, RED, KICK2>(k, a.poly, g, pin, pAin, pout, pAout, acc);
     else
-      gauge_site_f64<KICK, RED>(k, a.poly, g, pin, pAin, pout, pAout, acc);
+      gauge_site_f64<KICK, RED, KICK2>(k, a.poly, g, pin, pAin, pout, pAout, acc);
     if (KICK && act) {
       for (int q = 0; q < 2; ++q) store_out<NT>((P *)a.pi_out[q] + s, pout[q]);
       if (u1)
         for (int d = 0; d < 3; ++d) store_out<NT>((P *)a.piA_out[d] + s, pAout[d]);
     }
     if (RED && ((x + 1) % RG == 0 || (RAG && x + 1 == N))) {
-      double v[kNumRed] = {0, 0, acc[2], acc[0], acc[1], acc[3], acc[4], 0};
+      double v[kNumRed] = {acc[5], acc[6], acc[2], acc[0], acc[1], acc[3], acc[4], 0};
       if (!act)
-        for (int k2 = 2; k2 < 7; ++k2) v[k2] = 0.0;
+        for (int k2 = 0; k2 < 7; ++k2) v[k2] = 0.0;
       const size_t row = ((size_t)(x / RG) * nTy + ty) * nTz + tz;
       block_reduce_store_nt<kNumRed, 64 * GTY>(v, a.partials + row * kNumRed);
-      for (int k2 = 0; k2 < 5; ++k2) acc[k2] = 0.0;
+      for (int k2 = 0; k2 < 7; ++k2) acc[k2] = 0.0;
     }
     if (more) {
       if (KICK) {
@@ -287,6 +294,17 @@ template <bool F32, int GTY, int U1 = 0, bool RAG = false, bool NT = !RAG>
 hipError_t dispatch_tiled(bool drift, bool kick, bool red, const GaugePassArgs &a, int blocks, int XC, hipStream_t s)
 {
   const int G = gauge_rows_g((int)a.N);
+  if (a.ckick2 != 0.0) {
+    if constexpr (GTY == 4) {
+      if (!drift || !kick) return hipErrorInvalidValue;
+      if (red)
+        hipLaunchKernelGGL((k_gauge_tiled<F32, true, true, true, GTY, U1, RAG, NT, true>), dim3(blocks), dim3(64 * GTY), 0, s, a, XC, G);
+      else
+        hipLaunchKernelGGL((k_gauge_tiled<F32, true, true, false, GTY, U1, RAG, NT, true>), dim3(blocks), dim3(64 * GTY), 0, s, a, XC, G);
+      return hipGetLastError();
+    }
+    return hipErrorInvalidValue;
+  }
   const int code = (drift ? 4 : 0) | (kick ? 2 : 0) | (red ? 1 : 0);
 #define CLMI_GT(D, K, R)                                                                                  \
   case ((D ? 4 : 0) | (K ? 2 : 0) | (R ? 1 : 0)):                                                        \

@@ -151,8 +151,10 @@ __device__ __forceinline__ void apply_op(DevState *st, const double *red, const 
     case OP_KERNEL_ONLY:
       kernel = true;
       break;
-    case OP_VV_MOMENTA_KICK2:  // velocityverlet.h:249-256, scalar singlets only
-      b.pi2AvI = red[RED_PI2S_KICK2];
+    case OP_VV_MOMENTA_KICK2:  // velocityverlet.h:249-256
+      if (mc.ncs == 0) b.pi2AvI = red[RED_PI2S_KICK2];
+      if (mc.ncs > 0) b.CSpi2AvI = red[RED_PI2CS_KICK2];
+      if (mc.nu1 > 0) b.U1pi2AvI = red[RED_PI2U1_KICK2];
       break;
     case OP_VV_DRIFT_SF:  // velocityverlet.h:239-242
       b.aIM = b.aI;
