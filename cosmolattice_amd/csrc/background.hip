@@ -93,11 +93,13 @@ __global__ __launch_bounds__(kBlock) void k_gauss(const GaussArgs a)
   block_reduce_store<kNumRed>(v, a.partials + (size_t)blockIdx.x * kNumRed);
 }
 
-template <bool F32>
+// PAIRS: a thread takes two z-neighbours at a time and U pairs per turn, every load of them in flight: a load a
+// site and turn, with a division for its coordinates, ran at 2.7 TB/s (256^3 FP64 with the gradient 50 -> 35 us).  Pairs
+// do not straddle rows for even N only, and each is one access of two values: launch_means takes the one-site form for
+// odd N and for arrays that are not aligned to a pair.
+template <bool F32, bool PAIRS>
 __global__ __launch_bounds__(kBlock) void k_means(const MeansArgs a)
 {
-  // A thread takes two z-neighbours (N is even) at a time and U pairs per turn, every load of them in flight: a load a
-  // site and turn, with a division for its coordinates, ran at 2.7 TB/s (256^3 FP64 with the gradient 50 -> 35 us).
   constexpr int U = 2;
   double acc[3] = {0, 0, 0};
   struct Two {
@@ -117,7 +119,20 @@ __global__ __launch_bounds__(kBlock) void k_means(const MeansArgs a)
     if (F32) return (double)((const float *)a.p)[i] + (a.lo ? (double)a.lo[i] : 0.0);
     return ((const double *)a.p)[i];
   };
-  const uint32_t N = a.N, NN = N * N, pairs = a.V / 2, stride = gridDim.x * kBlock;
+  const uint32_t N = a.N, NN = N * N, pairs = PAIRS ? a.V / 2 : 0, stride = gridDim.x * kBlock;
+  if constexpr (!PAIRS)
+    for (uint32_t s = blockIdx.x * kBlock + threadIdx.x; s < a.V; s += stride) {
+      const double c = ld(s), v = c * a.scale;
+      acc[0] += v;
+      acc[1] += v * v;
+      if (a.grad) {
+        const uint32_t x = s / NN, y = (s - x * NN) / N, z = s - x * NN - y * N;
+        const double dx = ld(s - x * NN + (x + 1 == N ? 0 : x + 1) * NN) - c;
+        const double dy = ld(s - y * N + (y + 1 == N ? 0 : y + 1) * N) - c;
+        const double dz = ld(s - z + (z + 1 == N ? 0 : z + 1)) - c;
+        acc[2] += dx * dx + dy * dy + dz * dz;
+      }
+    }
   for (uint32_t i = blockIdx.x * kBlock + threadIdx.x; i < pairs; i += U * stride) {
     Two c[U], nx[U], ny[U];
     double nz[U];
@@ -331,10 +346,12 @@ hipError_t launch_gauss(const GaussArgs &a, int blocks, hipStream_t s)
 
 hipError_t launch_means(const MeansArgs &a, int blocks, hipStream_t s)
 {
+  const uintptr_t two = a.f32 ? sizeof(float2) : sizeof(double2);
+  const bool pairs = a.V % 2 == 0 && ((uintptr_t)a.p | (uintptr_t)a.lo) % two == 0;
   if (a.f32)
-    hipLaunchKernelGGL(k_means<true>, dim3(blocks), dim3(kBlock), 0, s, a);
+    hipLaunchKernelGGL((pairs ? k_means<true, true> : k_means<true, false>), dim3(blocks), dim3(kBlock), 0, s, a);
   else
-    hipLaunchKernelGGL(k_means<false>, dim3(blocks), dim3(kBlock), 0, s, a);
+    hipLaunchKernelGGL((pairs ? k_means<false, true> : k_means<false, false>), dim3(blocks), dim3(kBlock), 0, s, a);
   return hipGetLastError();
 }
 
