@@ -2280,13 +2280,16 @@ int autotune_gauge(clmi_ctx *c, int reps, std::string &rep)
   hipEvent_t e0, e1;
   HIPCHK(c, hipEventCreate(&e0));
   HIPCHK(c, hipEventCreate(&e1));
-  double best = 1e300, cur = 1e300;
-  int best_xc = c->gXC, best_blocks = c->blocks_g;
+  double best = 1e300, cur = 0.0;
+  int best_xc = c->gXC, best_blocks = c->blocks_g, last_blocks = 0;
   std::string lines;
   hipError_t e = hipSuccess;
-  for (int xc = 4; xc <= c->N && e == hipSuccess; xc *= 2) {
+  // the shortest x-chunk of every number of chunks (a longer one only makes the last chunk shorter), and the current one
+  for (int xc = 4; xc < c->N + 8 && e == hipSuccess; xc += 4) {
     int blocks = 0, rows = 0;
     if (!gauge_tiled_shape(c->N, c->gTY, xc, &blocks, &rows) || rows != c->rows_g) continue;
+    if (blocks == last_blocks && xc != c->gXC) continue;
+    last_blocks = blocks;
     auto launch = [&]() { return launch_gauge_tiled(c->f32, c->gTY, true, true, true, a, blocks, xc, stays_cached(c), c->stream); };
     e = launch();
     if (e == hipSuccess) e = hipEventRecord(e0, c->stream);
