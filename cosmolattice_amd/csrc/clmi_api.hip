@@ -2163,23 +2163,34 @@ int clmi_ensemble_autotune(clmi_ensemble *e, int reps, char *report, size_t repo
   EHIP(e, hipEventCreate(&t1));
   std::string rep;
   int rc = CLMI_OK;
+  auto chunk_name = [](const std::vector<RowsPlan> &plans) -> std::string {
+    if (plans.empty()) return "0";
+    for (const RowsPlan &rp : plans)
+      if (rp.XC != plans[0].XC) return "mixed";
+    return std::to_string(plans[0].XC);
+  };
   // Each group's batched fused pass from the current buffers into the spare ones (parity-0 table),
-  // timed per x-chunk; no parity flip and no background update, so the members' state is unchanged.
+  // timed with the members' current plans and per x-chunk; no parity flip and no background update, so the members'
+  // state is unchanged.
   for (size_t gi = 0; gi < e->groups.size() && rc == CLMI_OK; ++gi) {
     const clmi_ensemble::Group g0 = e->groups[gi];
     double best = 1e300;
     std::vector<RowsPlan> best_plans;
     std::string line = "# group VZ=" + std::to_string(g0.vz) + " members=" + std::to_string(g0.count);
-    for (int xc : {8, 16, 32, 64}) {
+    std::vector<RowsPlan> now;
+    for (int i = g0.first; i < g0.first + g0.count; ++i) now.push_back(e->order[i]->rplan);
+    for (int xc : {0, 8, 16, 24, 32, 64}) {  // 0: the members' current plans
       std::vector<RowsPlan> plans;
-      bool ok = true;
+      bool ok = true, same = xc != 0;  // same: an x-chunk that every member has already
       for (int i = g0.first; i < g0.first + g0.count && ok; ++i) {
         const clmi_ctx *c = e->order[i];
-        RowsPlan rp;
-        ok = scalar_rows_plan(c->N, c->cfg.n_scalars, c->f32, xc, c->rplan.MM, rows_shape(c->cfg.flags), &rp);
+        RowsPlan rp = now[i - g0.first];
+        same = same && rp.XC == xc;
+        if (xc)
+          ok = scalar_rows_plan(c->N, c->cfg.n_scalars, c->f32, xc, rp.MM, rows_shape(c->cfg.flags), &rp);
         plans.push_back(rp);
       }
-      if (!ok) continue;
+      if (!ok || same) continue;
       for (int i = g0.first; i < g0.first + g0.count; ++i) e->order[i]->rplan = plans[i - g0.first];
       if ((rc = ens_tables(e)) != CLMI_OK) break;
       const clmi_ensemble::Group &g = e->groups[gi];
@@ -2199,7 +2210,7 @@ int clmi_ensemble_autotune(clmi_ensemble *e, int reps, char *report, size_t repo
         break;
       }
       const double us = 1e3 * ms / reps;
-      line += " XC=" + std::to_string(xc) + ":" + std::to_string(us);
+      line += " XC=" + chunk_name(plans) + ":" + std::to_string(us);
       if (us < best) {
         best = us;
         best_plans = plans;
@@ -2207,7 +2218,7 @@ int clmi_ensemble_autotune(clmi_ensemble *e, int reps, char *report, size_t repo
     }
     if (rc == CLMI_OK && !best_plans.empty())
       for (int i = g0.first; i < g0.first + g0.count; ++i) e->order[i]->rplan = best_plans[i - g0.first];
-    rep += line + " -> XC=" + std::to_string(best_plans.empty() ? 0 : best_plans[0].XC) + "\n";
+    rep += line + " -> XC=" + chunk_name(best_plans) + "\n";
   }
   (void)hipEventDestroy(t0);
   (void)hipEventDestroy(t1);

@@ -5,7 +5,8 @@ import re
 import numpy as np
 import pytest
 
-from cosmolattice_amd.clmi import (CLMI_F32_BULK, CLMI_F64, FLD_CS, FLD_U1, PI_CS, PI_U1, Lattice, lphi4U1)
+from cosmolattice_amd.clmi import (CLMI_F32_BULK, CLMI_F64, FLD_CS, FLD_S, FLD_U1, PI_CS, PI_S, PI_U1, Ensemble,
+                                   Lattice, lphi4, lphi4U1)
 from test_gpu_parity import say
 
 pytestmark = pytest.mark.gpu
@@ -43,3 +44,30 @@ def test_autotune_times_the_ragged_u1_default(gpu, N, prec):
     assert res[0][1] == res[1][1]
     for a, b in zip(res[0][0], res[1][0]):
         assert np.array_equal(a, b)
+
+
+@pytest.mark.parametrize("prec", [CLMI_F64, CLMI_F32_BULK])
+def test_ensemble_autotune_times_the_members_plans(gpu, prec):
+    """Each size class's current x-chunk (24 at 192^3) is among those timed, and the one chosen was timed fastest."""
+    say(f"case ensemble autotune prec={prec}")
+    spec = lphi4(100.0, phi0_gev=5.6964e18, lam=1.0, pi0_program=-0.5)
+    rng = np.random.default_rng(1)
+    members = []
+    for N in (64, 64, 128, 192):
+        lat = Lattice(spec, N, 0.4909, 0.005, prec, expansion=False)
+        for k in (FLD_S, PI_S):
+            for f in range(2):
+                lat.upload(k, f, 0, 0.3 * rng.standard_normal((N, N, N)))
+        members.append(lat)
+    chunks = {N: re.search(r" XC=(\d+)", lat.plan()).group(1) for N, lat in zip((64, 64, 128, 192), members)}
+    ens = Ensemble(members)
+    rep = ens.autotune(2)
+    say(f"defaults {chunks}\n{rep}")
+    for line, N in zip(rep.strip().splitlines(), (64, 128, 192)):
+        timed = {x: float(us) for x, us in re.findall(r"XC=(\d+):([\d.]+)", line)}
+        chosen = line.split("-> XC=")[1]
+        assert chunks[N] in timed
+        assert timed[chosen] == min(timed.values())
+    ens.close()
+    for lat in members:
+        lat.close()
