@@ -14,6 +14,7 @@
 
 #include <algorithm>
 #include <atomic>
+#include <chrono>
 #include <climits>
 #include <cstddef>
 #include <cmath>
@@ -74,7 +75,9 @@ struct clmi_ctx {
   ResidentPlan resp;
   uint64_t *res_lines = nullptr;
   void *res_xch = nullptr;
-  int *res_err = nullptr;  // page-locked, device-visible
+  ResidentGate *res_gate = nullptr;
+  ResidentHost *res_host = nullptr;  // page-locked, device-visible
+  uint32_t res_arrived = 0, res_word = 0;  // of the gate, as the last launch left it
 
   // large downloads (host_read) and the adjoint's seeds; allocated at the first use
   char *bounce = nullptr;  // page-locked, kBounceSlots chunks
@@ -215,13 +218,13 @@ int prof_event(clmi_ctx *c)
   return CLMI_OK;
 }
 
-// Wait for the stream, then report a resident evolver whose workgroups lost each other (its launch leaves the
-// arrays it read untouched and writes no result).
+// Wait for the stream, then report a resident evolver whose workgroups lost each other after all had started, which
+// takes a device that stops in the middle of a launch: the context's state is lost then, for good.
 int sync_stream(clmi_ctx *c)
 {
   HIPCHK(c, hipStreamSynchronize(c->stream));
-  if (c->res_err && __atomic_load_n(c->res_err, __ATOMIC_RELAXED) != 0)
-    return fail(c, CLMI_E_HIP, "the resident evolver's workgroups timed out waiting for each other");
+  if (c->res_host && __atomic_load_n(&c->res_host->lost, __ATOMIC_RELAXED) != 0)
+    return fail(c, CLMI_E_HIP, "the resident evolver's workgroups lost each other; the context's state is lost");
   return CLMI_OK;
 }
 
@@ -482,11 +485,32 @@ int pass_update(clmi_ctx *c, bool drift, bool kick, bool red, double cdt_s, doub
 // 15 us a pass; 128^3 two fields FP64: 47 us, 17.7 against 37 us).
 constexpr int kResMinPasses = 4;
 
+// Waits until the gate of the resident launch just queued is decided; whether it opened.  The launch's workgroups decide
+// it when they start, so the call returns while they evolve the lattice (work queued before them comes first).
+int resident_opened(clmi_ctx *c, uint32_t shut, bool *opened)
+{
+  const auto t0 = std::chrono::steady_clock::now();
+  for (bool ended = false;; ) {
+    const uint32_t w = __atomic_load_n(&c->res_host->word, __ATOMIC_RELAXED);
+    if (w != shut) {
+      *opened = w == shut + 1;
+      return CLMI_OK;
+    }
+    if (ended) return fail(c, CLMI_E_HIP, "a resident launch ended without opening or closing its gate");
+    if (std::chrono::steady_clock::now() - t0 < std::chrono::microseconds(200)) continue;
+    std::this_thread::sleep_for(std::chrono::microseconds(20));
+    const hipError_t e = hipStreamQuery(c->stream);
+    if (e != hipErrorNotReady) HIPCHK(c, e);
+    ended = e == hipSuccess;
+  }
+}
+
 // Runs `passes` passes of a scheme as one launch of the resident evolver, where the lattice has a plan for it:
 // drift + kick passes (RES_LF), double-kick passes (RES_VV) or pairs of drift + kick and drift (RES_PV).
 // *done = false: not taken (nothing was changed), the caller runs the passes one by one, which gives the
 // same bits.  Not taken: too few passes for the cooperative launch to pay, pass timing on, a background snapshot
-// asked for, more weights than its arguments hold, no memory for its buffers, or a device too small for its tiles.
+// asked for, more weights than its arguments hold, no memory for its buffers, a launch that the device refuses, or
+// a gate that closed because the workgroups did not all find room; after the last two the context does not try again.
 int run_resident(clmi_ctx *c, int scheme, int passes, const double *ws, int nws, bool *done)
 {
   *done = false;
@@ -497,16 +521,20 @@ int run_resident(clmi_ctx *c, int scheme, int passes, const double *ws, int nws,
   if (!c->res_lines) {
     const size_t xb = 2 * (size_t)nf * c->V * bytes_field(c->f32);
     if (hipMalloc(&c->res_lines, line_bytes) != hipSuccess || hipMalloc(&c->res_xch, xb) != hipSuccess ||
-        hipHostMalloc((void **)&c->res_err, sizeof(int), hipHostMallocMapped) != hipSuccess) {
+        hipMalloc(&c->res_gate, sizeof(ResidentGate)) != hipSuccess ||
+        hipHostMalloc((void **)&c->res_host, sizeof(ResidentHost), hipHostMallocMapped | hipHostMallocCoherent) != hipSuccess) {
       (void)hipGetLastError();
       c->resident = false;  // a small lattice that cannot have them runs pass by pass
       if (c->res_lines) (void)hipFree(c->res_lines);
       if (c->res_xch) (void)hipFree(c->res_xch);
+      if (c->res_gate) (void)hipFree(c->res_gate);
       c->res_lines = nullptr;
       c->res_xch = nullptr;
+      c->res_gate = nullptr;
       return CLMI_OK;
     }
-    *c->res_err = 0;
+    *c->res_host = ResidentHost{};
+    HIPCHK(c, hipMemsetAsync(c->res_gate, 0, sizeof(ResidentGate), c->stream));
     c->res_epoch = UINT32_MAX;  // clears the lines below
   }
   if (UINT32_MAX - c->res_epoch <= (uint32_t)passes) {
@@ -525,14 +553,24 @@ int run_resident(clmi_ctx *c, int scheme, int passes, const double *ws, int nws,
   r.lines = c->res_lines;
   r.xch = c->res_xch;
   r.epoch0 = c->res_epoch;
-  r.err = c->res_err;
-  const hipError_t e = launch_scalar_resident(scheme, nf, c->f32, poly_kind(c->spoly, nf), c->resp, r, c->stream);
-  if (e == hipErrorCooperativeLaunchTooLarge) {
+  r.refuse = (c->cfg.flags & CLMI_FLAG_REFUSE_RESIDENT) != 0;
+  r.gate = c->res_gate;
+  r.host = c->res_host;
+  r.arrived = c->res_arrived + (uint32_t)tiles;
+  r.shut = c->res_word;
+  if (launch_scalar_resident(scheme, nf, c->f32, poly_kind(c->spoly, nf), c->resp, r, c->stream) != hipSuccess) {
     (void)hipGetLastError();
     c->resident = false;
     return CLMI_OK;
   }
-  HIPCHK(c, e);
+  bool opened = false;
+  CHK(resident_opened(c, r.shut, &opened));
+  c->res_arrived = r.arrived;
+  c->res_word = c->res_host->word;
+  if (!opened) {
+    c->resident = false;
+    return CLMI_OK;
+  }
   c->res_epoch += (uint32_t)passes;
   c->cur_fS = 1 - c->cur_fS;
   c->cur_pS = 1 - c->cur_pS;
@@ -835,7 +873,8 @@ void clmi_destroy(clmi_ctx *c)
   if (c->done_count) (void)hipFree(c->done_count);
   if (c->res_lines) (void)hipFree(c->res_lines);
   if (c->res_xch) (void)hipFree(c->res_xch);
-  if (c->res_err) (void)hipHostFree(c->res_err);
+  if (c->res_gate) (void)hipFree(c->res_gate);
+  if (c->res_host) (void)hipHostFree(c->res_host);
   if (c->dstate) (void)hipFree(c->dstate);
   if (c->stage) (void)hipFree(c->stage);
   if (c->fk) (void)hipFree(c->fk);
@@ -2156,7 +2195,8 @@ int clmi_ensemble_autotune(clmi_ensemble *e, int reps, char *report, size_t repo
   if (report && report_len) report[0] = '\0';
   if (reps < 1) reps = 1;
   EHIP(e, hipSetDevice(e->device));
-  for (clmi_ctx *c : e->m) EHIP(e, hipStreamSynchronize(c->stream));
+  for (clmi_ctx *c : e->m)
+    if (sync_stream(c) != CLMI_OK) return efail(e, CLMI_E_HIP, "member: " + c->err);
   CHK(ens_tables(e));
   hipEvent_t t0 = nullptr, t1 = nullptr;
   EHIP(e, hipEventCreate(&t0));
@@ -2247,7 +2287,8 @@ int clmi_ensemble_lf_evolve(clmi_ensemble *e, int nsteps)
     }
     --nsteps;
   }
-  for (clmi_ctx *c : e->m) EHIP(e, hipStreamSynchronize(c->stream));
+  for (clmi_ctx *c : e->m)
+    if (sync_stream(c) != CLMI_OK) return efail(e, CLMI_E_HIP, "member: " + c->err);
   CHK(ens_tables(e));
   // two steps (both buffer parities) of every group per graph replay
   if (nsteps >= 2 && !e->exec) CHK(ens_capture(e));

@@ -263,6 +263,13 @@ hipError_t launch_update_batch(const UpdMember *d_members, int n, const UpdateOp
 constexpr int kResThreads = 512;
 constexpr int kResMaxWeights = 16;  // composition weights
 enum ResScheme : int { RES_LF = 0, RES_VV = 1, RES_PV = 2 };
+struct ResidentGate {  // device
+  uint32_t arrived, word;
+};
+struct ResidentHost {  // page-locked, written by the device
+  uint32_t word;       // the gate's, once it is decided
+  int lost;            // a wait between workgroups ran out
+};
 struct ResidentArgs {
   ScalarPassArgs a;  // current arrays (in) and where the final ones go (out); a.cdt, a.ckick unused
   DevState *st;
@@ -274,8 +281,11 @@ struct ResidentArgs {
   uint64_t *lines;     // 2 x 8 x tiles words: partial sums with the epoch of their pass
   void *xch;           // 2 x n_scalars x V momenta: boundary values of the last two kicks
   uint32_t epoch0;     // passes of earlier launches on these buffers
-  int pad;
-  int *err;            // host-visible: a wait between workgroups ran out
+  int refuse;          // the gate stays shut (testing)
+  ResidentGate *gate;
+  ResidentHost *host;
+  uint32_t arrived;    // workgroups that have arrived at the gate once all of this launch have
+  uint32_t shut;       // the gate's word before this launch; shut + 1: open, shut + 2: closed for good
 };
 // Tiles of the resident evolver for an N^3 lattice: chunks of kResThreads * VZ sites of a plane by P planes.
 struct ResidentPlan {
@@ -283,7 +293,7 @@ struct ResidentPlan {
   bool ragged = false;  // some tiles may not be full
 };
 bool resident_plan(int N, int nf, ResidentPlan *p);
-// hipErrorCooperativeLaunchTooLarge where the device does not hold all tiles at once.
+// An error where the device does not hold all tiles at once (hipErrorCooperativeLaunchTooLarge) or has no such launches.
 hipError_t launch_scalar_resident(int scheme, int nf, bool f32, int pk, const ResidentPlan &p, const ResidentArgs &r, hipStream_t s);
 
 // ---- adjoint (adjoint_kernels.hip) ----

@@ -20,8 +20,12 @@
 // written back or invalidated.  Buffers alternate by parity: a workgroup can reach epoch e + 2 only after all
 // have written epoch e + 1, which they do after their last read of epoch e.
 //
-// The launch is cooperative, so all workgroups are resident together; a wait that sees no progress for
-// kSpinLimit polls sets the error word and ends (no output is written then), so the grid always drains.
+// The launch is cooperative, but that check knows nothing of what else holds the device's CUs (another process's
+// launch of this kind may wait for ours), so a workgroup first arrives at a gate.  The last to arrive opens it; one
+// that waits there for kGateLimit polls (about a second) closes it, whichever comes first, and the host learns which.
+// Nothing is written before the gate, so a closed one costs the wait alone: the host runs the same passes one by
+// one.  Behind an open gate every workgroup is on the chip and every wait ends; kSpinLimit is there so that
+// the grid drains even if the device itself fails, and the state is lost then (the host reports it).
 //
 // Measured (MI355X, us per leapfrog pass, resident against pass and update launches; VV2 in brackets):
 //   64^3  one field  FP64 6.0 / 15.0 (6.6 / 16.6)    two fields FP32-bulk 7.3 / 18.2 (7.8 / 19.8)
@@ -44,7 +48,30 @@
 namespace clmi {
 namespace {
 
-constexpr int kSpinLimit = 1 << 22;
+constexpr int kSpinLimit = 1 << 22, kGateLimit = 1 << 20;
+
+__device__ __forceinline__ void decide_gate(const ResidentArgs &r, uint32_t want)
+{
+  uint32_t was = r.shut;
+  if (__hip_atomic_compare_exchange_strong(&r.gate->word, &was, want, __ATOMIC_RELAXED, __ATOMIC_RELAXED,
+                                           __HIP_MEMORY_SCOPE_AGENT))
+    __hip_atomic_store(&r.host->word, want, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_SYSTEM);
+}
+// By one thread of every workgroup: arrive, and (later) wait for the decision; whether the gate opened.
+__device__ __forceinline__ void arrive_at_gate(const ResidentArgs &r)
+{
+  const uint32_t n = __hip_atomic_fetch_add(&r.gate->arrived, 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) + 1;
+  if (r.refuse) decide_gate(r, r.shut + 2);
+  else if (n == r.arrived) decide_gate(r, r.shut + 1);
+}
+__device__ __forceinline__ bool pass_gate(const ResidentArgs &r)
+{
+  for (int spin = 0;; ++spin) {
+    const uint32_t w = __hip_atomic_load(&r.gate->word, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+    if (w != r.shut) return w == r.shut + 1;
+    if (spin >= kGateLimit) decide_gate(r, r.shut + 2);  // (or somebody else has by now: the next poll shows it)
+  }
+}
 
 __device__ __forceinline__ void xstore64(uint64_t *p, uint64_t v)
 {
@@ -293,9 +320,9 @@ __global__ __launch_bounds__(kResThreads) void k_scalar_resident(const ResidentA
   auto has = [&](int p) -> bool { return !RAG || p >= pf; };
 
   if (tid == 0) {
+    arrive_at_gate(r);
     S = *r.st;
     MC = r.mc;
-    dead = 0;
   }
 
   V phi[P][NF][VZ];
@@ -361,7 +388,9 @@ __global__ __launch_bounds__(kResThreads) void k_scalar_resident(const ResidentA
       else yhp[j][k] = q[k];
     }
   }
+  if (tid == 0) dead = !pass_gate(r);
   __syncthreads();
+  if (dead) return;
 
   const bool red = r.mc.expansion != 0;
   const double dt = r.mc.dt;
@@ -547,7 +576,7 @@ __global__ __launch_bounds__(kResThreads) void k_scalar_resident(const ResidentA
     for (int k = 0; k < NS; ++k) v[k] = wave_sum(v[k]);
     __syncthreads();  // every tile's words seen; wsum free
     if (dead) {
-      if (tid == 0) __hip_atomic_store(r.err, 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_SYSTEM);
+      if (tid == 0) __hip_atomic_store(&r.host->lost, 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_SYSTEM);
       return false;
     }
     if (lane == 0)

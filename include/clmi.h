@@ -57,6 +57,10 @@ extern "C" {
  * the next run in one pass (they read the same fields with the same coefficients); the results are
  * bit-identical either way.  It also turns the resident evolver off.  The flag exists for testing. */
 #define CLMI_FLAG_NO_DOUBLE_KICK 32
+/* clmi_config.flags: every launch of the resident evolver finds its gate closed, as where its workgroups cannot
+ * all start on a shared device; the passes then run one by one, with the same results.  The flag exists for
+ * testing. */
+#define CLMI_FLAG_REFUSE_RESIDENT 64
 /* clmi_config.flags: memory mode m of the full-row lattice pass (0 = the library's default: ordinary
  * accesses where both buffers of the state fit the 256 MB last-level cache (64^3 to 192^3), else 1; 1 =
  * non-temporal stores, 3 = also non-temporal loads of the momenta, 7 = also of the workgroup's own
