@@ -279,7 +279,7 @@ struct ResidentArgs {
   double ws[kResMaxWeights];
   int groups, chunks;  // tiles along x and within a plane
   uint64_t *lines;     // 2 x 8 x tiles words: partial sums with the epoch of their pass
-  void *xch;           // 2 x n_scalars x V momenta: boundary values of the last two kicks
+  void *xch[2];        // n_scalars x V momenta each: boundary values of the last two kicks (the out arrays)
   uint32_t epoch0;     // passes of earlier launches on these buffers
   int refuse;          // the gate stays shut (testing)
   ResidentGate *gate;

@@ -18,7 +18,9 @@
 // words after the barrier that follows every thread's wait for its own momentum stores, and
 // all exchanged data goes through agent-scope accesses, which bypass the incoherent L2s; no cache is
 // written back or invalidated.  Buffers alternate by parity: a workgroup can reach epoch e + 2 only after all
-// have written epoch e + 1, which they do after their last read of epoch e.
+// have written epoch e + 1, which they do after their last read of epoch e.  They are the arrays that take the
+// final state: a workgroup stores that when it has seen every workgroup's words of the last pass, after which nobody
+// reads or writes exchanged momenta.
 //
 // The launch is cooperative, but that check knows nothing of what else holds the device's CUs (another process's
 // launch of this kind may wait for ours), so a workgroup first arrives at a gate.  The last to arrive opens it; one
@@ -407,9 +409,9 @@ __global__ __launch_bounds__(kResThreads) void k_scalar_resident(const ResidentA
     const uint32_t epoch = r.epoch0 + 1 + (uint32_t)m;
     const bool last = m + 1 == r.passes;
     // momenta of this kick, or of the last one (position Verlet's drift passes): alternate buffers
-    const uint32_t xsize = (uint32_t)NF * a.V;
+    const bool odd = ((SCH == RES_PV ? m >> 1 : m) & 1) != 0;
     const __amdgpu_buffer_rsrc_t xb = __builtin_amdgcn_make_buffer_rsrc(
-        (M *)r.xch + (size_t)((SCH == RES_PV ? m >> 1 : m) & 1) * xsize, 0, (int)(xsize * (uint32_t)sizeof(M)), 0x00027000);
+        odd ? r.xch[1] : r.xch[0], 0, (int)((uint32_t)NF * a.V * (uint32_t)sizeof(M)), 0x00027000);
     const double fs = S.fdrift_s;
     const SiteK kc = site_consts(ck, ck2, S.aK, S.aV, a.inv_dx, a.inv_dx2);
     const int ft = fresh(tid);
