@@ -1669,6 +1669,8 @@ AdjFields adj_view_cur(const clmi_ctx *c)
   return v;
 }
 
+constexpr size_t kSideSeeds = (size_t)2 << 20;
+
 struct AdjRun {
   clmi_ctx *c = nullptr;
   std::vector<AdjState> checkpoints, segment;
@@ -1776,14 +1778,17 @@ int clmi_adjoint_lf(clmi_ctx *c, int nsteps, int checkpoint_every, int bg_from_f
   c->snap = run.tape + nsteps;
   CHK(flush(c));
   c->snap = nullptr;
-  // the seeds come up on a stream of their own while the forward run computes
-  if (!c->side) HIPCHK(c, hipStreamCreateWithFlags(&c->side, hipStreamNonBlocking));
+  // The seeds come up on a stream of their own while the forward run computes, from kSideSeeds on: 20 steps, two fields,
+  // with / without it 100^3 FP64 9.1 / 12.4 ms, 64^3 3.0 / 3.8, 48^3 (3.5 MB) 1.88 / 1.93.  At 32^3 (1 MB) more than half
+  // the runs lose 0.35 ms to the second stream (1.76 / 1.55), where 24^3 gains 0.04.
+  const bool aside = sizeof(double) * 2 * nf * c->V >= kSideSeeds;
+  if (aside && !c->side) HIPCHK(c, hipStreamCreateWithFlags(&c->side, hipStreamNonBlocking));
+  const hipStream_t up = aside ? c->side : c->stream;
   for (int f = 0; f < nf; ++f) {
-    HIPCHK(c, hipMemcpyAsync(run.lam + (size_t)f * c->V, seed_fld[f], sizeof(double) * c->V, hipMemcpyHostToDevice, c->side));
-    HIPCHK(c, hipMemcpyAsync(run.lam + (size_t)(nf + f) * c->V, seed_pi[f], sizeof(double) * c->V, hipMemcpyHostToDevice,
-                             c->side));
+    HIPCHK(c, hipMemcpyAsync(run.lam + (size_t)f * c->V, seed_fld[f], sizeof(double) * c->V, hipMemcpyHostToDevice, up));
+    HIPCHK(c, hipMemcpyAsync(run.lam + (size_t)(nf + f) * c->V, seed_pi[f], sizeof(double) * c->V, hipMemcpyHostToDevice, up));
   }
-  HIPCHK(c, hipStreamSynchronize(c->side));
+  if (aside) HIPCHK(c, hipStreamSynchronize(c->side));
   HIPCHK(c, hipMemcpyAsync(tape.data(), run.tape, sizeof(clmi_background) * (size_t)(nsteps + 1),
                            hipMemcpyDeviceToHost, c->stream));
   CHK(sync_stream(c));
