@@ -142,13 +142,21 @@ size_t bytes_field(bool f32) { return f32 ? 4 : 8; }
 
 // Row-pass shape selector from clmi_config.flags (bit 0: VZ = 4 rows, bit 1: 4-row tiles).
 // Memory mode of the full-row pass when neither the configuration nor clmi_autotune chooses one, for a state of `bytes` in
-// both of its buffers: ordinary accesses where it stays in the 256 MB last-level cache from step to step, else
-// non-temporal stores.  A leapfrog step, modes 0 / 1 / 15: 128^3 two fields FP32-bulk (100 MB) 24.1 / 30.0 / 31.0 us and
-// FP64 (134 MB) 27.8 / 32.5 / 33.9, 192^3 one field FP64 (226 MB) 43.5 / 56 / 61; past the cache 192^3 two fields
-// FP32-bulk (340 MB) 86.5 / 82.7 / 84.4 and FP64 (453 MB) 124 / 112 / 123, 256^3 FP32-bulk 181 / 177 / 174, 512^3 - / 1457 /
-// 1510 to 1700.
+// both of its buffers, by what of it the 256 MB last-level cache keeps from pass to pass.
+//  - Both buffers fit: ordinary accesses.  A leapfrog step, modes 0 / 1 / 15: 128^3 two fields FP32-bulk (100 MB) 24.1 / 30.0
+//    / 31.0 us and FP64 (134 MB) 27.8 / 32.5 / 33.9, 192^3 one field FP64 (226 MB) 43.5 / 56 / 61.
+//  - One buffer fits: non-temporal stores alone, modes 1 / 3 / 15: 192^3 two fields FP32-bulk (340 MB) 84 / 88 / 88 and FP64
+//    (453 MB) 110 / 125 / 125; the averages of 256^3 one field FP32-bulk (403 MB) 52 / 56 / 57, its step 88 / 89 / 88.
+//  - One buffer is up to twice the cache: loads that pass the cache by (mode 15) leave in it what the next pass reads.
+//    256^3 two fields FP32-bulk (805 MB): a step is the same (172.2 / 173.6 / 171.6 and, in other memory, 170.2 / 169.8 /
+//    171.0), the averages 99 / 82 / 81, a velocity-Verlet step by itself 289 / 276 / 278.
+//  - Beyond, nothing is kept: 512^3 1467 / 1573 / 1630.
 constexpr double kCacheBytes = 256.0 * 1048576.0;
-int default_mem_mode(double bytes) { return bytes <= kCacheBytes ? 0 : 1; }
+int default_mem_mode(double bytes)
+{
+  if (bytes <= kCacheBytes) return 0;
+  return bytes > 2 * kCacheBytes && bytes <= 4 * kCacheBytes ? 15 : 1;
+}
 
 int rows_shape(int flags)
 {

@@ -62,8 +62,8 @@ extern "C" {
  * testing. */
 #define CLMI_FLAG_REFUSE_RESIDENT 64
 /* clmi_config.flags: memory mode m of the full-row lattice pass (0 = the library's default: ordinary
- * accesses where both buffers of the state fit the 256 MB last-level cache (64^3 to 192^3), else 1; 1 =
- * non-temporal stores, 3 = also non-temporal loads of the momenta, 7 = also of the workgroup's own
+ * accesses where both buffers of the state fit the 256 MB last-level cache (64^3 to 192^3), 15 where one buffer
+ * takes one to two times the cache (two fields at 256^3), else 1; 1 = non-temporal stores, 3 = also non-temporal loads of the momenta, 7 = also of the workgroup's own
  * field rows, 15 = as 7 but ordinary loads for the tile's first and last rows).  Results do not
  * depend on it; clmi_autotune chooses one.  This flag, like the shape flags, also selects the
  * full-row pass where another pass is the default (FP64 at 256^3 runs the tiled pass). */
