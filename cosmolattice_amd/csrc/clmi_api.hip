@@ -78,6 +78,12 @@ struct clmi_ctx {
   ResidentGate *res_gate = nullptr;
   ResidentHost *res_host = nullptr;  // page-locked, device-visible
   uint32_t res_arrived = 0, res_word = 0;  // of the gate, as the last launch left it
+  DevState *res_closed = nullptr;
+  struct {  // the last resident launch, until its gate is known to have opened (settle)
+    bool on = false;
+    int scheme = 0, passes = 0, nws = 0, f = 0, p = 0;  // f, p: buffers that take its final state
+    double ws[kResMaxWeights] = {};
+  } res_last;
 
   // large downloads (host_read) and the adjoint's seeds; allocated at the first use
   char *bounce = nullptr;  // page-locked, kBounceSlots chunks
@@ -510,32 +516,13 @@ int pass_update(clmi_ctx *c, bool drift, bool kick, bool red, double cdt_s, doub
 // 15 us a pass; 128^3 two fields FP64: 47 us, 17.7 against 37 us).
 constexpr int kResMinPasses = 4;
 
-// Waits until the gate of the resident launch just queued is decided; whether it opened.  The launch's workgroups decide
-// it when they start, so the call returns while they evolve the lattice (work queued before them comes first).
-int resident_opened(clmi_ctx *c, uint32_t shut, bool *opened)
-{
-  const auto t0 = std::chrono::steady_clock::now();
-  for (bool ended = false;; ) {
-    const uint32_t w = __atomic_load_n(&c->res_host->word, __ATOMIC_RELAXED);
-    if (w != shut) {
-      *opened = w == shut + 1;
-      return CLMI_OK;
-    }
-    if (ended) return fail(c, CLMI_E_HIP, "a resident launch ended without opening or closing its gate");
-    if (std::chrono::steady_clock::now() - t0 < std::chrono::microseconds(200)) continue;
-    std::this_thread::sleep_for(std::chrono::microseconds(20));
-    const hipError_t e = hipStreamQuery(c->stream);
-    if (e != hipErrorNotReady) HIPCHK(c, e);
-    ended = e == hipSuccess;
-  }
-}
-
 // Runs `passes` passes of a scheme as one launch of the resident evolver, where the lattice has a plan for it:
 // drift + kick passes (RES_LF), double-kick passes (RES_VV) or pairs of drift + kick and drift (RES_PV).
 // *done = false: not taken (nothing was changed), the caller runs the passes one by one, which gives the
 // same bits.  Not taken: too few passes for the cooperative launch to pay, pass timing on, a background snapshot
-// asked for, more weights than its arguments hold, no memory for its buffers, a launch that the device refuses, or
-// a gate that closed because the workgroups did not all find room; after the last two the context does not try again.
+// asked for, more weights than its arguments hold, no memory for its buffers, or a launch that the device refuses (after
+// which the context does not try again).  Whether the launch's gate opened is found out by the context's next call
+// (settle), so that calls on several contexts still queue their work without waiting for one another.
 int run_resident(clmi_ctx *c, int scheme, int passes, const double *ws, int nws, bool *done)
 {
   *done = false;
@@ -546,13 +533,16 @@ int run_resident(clmi_ctx *c, int scheme, int passes, const double *ws, int nws,
   if (!c->res_lines) {
     if (hipMalloc(&c->res_lines, line_bytes) != hipSuccess ||
         hipMalloc(&c->res_gate, sizeof(ResidentGate)) != hipSuccess ||
+        hipMalloc(&c->res_closed, sizeof(DevState)) != hipSuccess ||
         hipHostMalloc((void **)&c->res_host, sizeof(ResidentHost), hipHostMallocMapped | hipHostMallocCoherent) != hipSuccess) {
       (void)hipGetLastError();
       c->resident = false;  // a small lattice that cannot have them runs pass by pass
       if (c->res_lines) (void)hipFree(c->res_lines);
       if (c->res_gate) (void)hipFree(c->res_gate);
+      if (c->res_closed) (void)hipFree(c->res_closed);
       c->res_lines = nullptr;
       c->res_gate = nullptr;
+      c->res_closed = nullptr;
       return CLMI_OK;
     }
     *c->res_host = ResidentHost{};
@@ -579,6 +569,7 @@ int run_resident(clmi_ctx *c, int scheme, int passes, const double *ws, int nws,
   r.refuse = (c->cfg.flags & CLMI_FLAG_REFUSE_RESIDENT) != 0;
   r.gate = c->res_gate;
   r.host = c->res_host;
+  r.closed_st = c->res_closed;
   r.arrived = c->res_arrived + (uint32_t)tiles;
   r.shut = c->res_word;
   if (launch_scalar_resident(scheme, nf, c->f32, poly_kind(c->spoly, nf), c->resp, r, c->stream) != hipSuccess) {
@@ -586,19 +577,114 @@ int run_resident(clmi_ctx *c, int scheme, int passes, const double *ws, int nws,
     c->resident = false;
     return CLMI_OK;
   }
-  bool opened = false;
-  CHK(resident_opened(c, r.shut, &opened));
   c->res_arrived = r.arrived;
-  c->res_word = c->res_host->word;
-  if (!opened) {
-    c->resident = false;
-    return CLMI_OK;
-  }
   c->res_epoch += (uint32_t)passes;
   c->cur_fS = 1 - c->cur_fS;
   c->cur_pS = 1 - c->cur_pS;
+  auto &l = c->res_last;
+  l.on = true;
+  l.scheme = scheme;
+  l.passes = passes;
+  l.nws = nws;
+  l.f = c->cur_fS;
+  l.p = c->cur_pS;
+  for (int i = 0; i < nws; ++i) l.ws[i] = ws[i];
   *done = true;
   return CLMI_OK;
+}
+
+// A leapfrog step after the first: the deferred drift, and the kick of weight w.
+int lf_pass(clmi_ctx *c, double w)
+{
+  const bool ex = c->cfg.expansion != 0;
+  const double dt = c->cfg.dt;
+  return pass_update(c, true, true, ex, dt, w * dt, w * dt, ex, {{OP_STORE_FIELDS, 0.0}, {OP_LF_MOMENTA, 0.0}});
+}
+
+double stage_weight(const double *ws, int nws, int s) { return ws[s < nws ? s : 2 * nws - 2 - s]; }
+
+// Velocity-Verlet stages k0 to K - 1 by double-kick passes, the last by one with a single kick.
+int vv_passes(clmi_ctx *c, const double *ws, int nws, int k0, int K)
+{
+  const bool ex = c->cfg.expansion != 0;
+  const double dt = c->cfg.dt;
+  const int stages = 2 * nws - 1;
+  for (int k = k0; k < K; ++k) {
+    const double w = stage_weight(ws, nws, k % stages);
+    if (k + 1 < K) {
+      const double w2 = stage_weight(ws, nws, (k + 1) % stages);
+      CHK(pass_update(c, true, true, ex, dt * w, w * dt / 2, dt / 2 * w, ex,
+                      {{OP_STORE_FIELDS, 0.0}, {OP_VV_MOMENTA, 0.0}, {OP_VV_SF_ONE, w}, {OP_VV_SF_HALF, w2},
+                       {OP_VV_MOMENTA_KICK2, 0.0}, {OP_VV_DRIFT_SF, w2}},
+                      w2 * dt / 2, dt / 2 * w2));
+    } else {
+      CHK(pass_update(c, true, true, ex, dt * w, w * dt / 2, dt / 2 * w, ex,
+                      {{OP_STORE_FIELDS, 0.0}, {OP_VV_MOMENTA, 0.0}, {OP_VV_SF_ONE, w}}));
+    }
+  }
+  return CLMI_OK;
+}
+
+// nsteps position-Verlet steps whose first scale-factor drift has run.
+int pv_passes(clmi_ctx *c, const double *ws, int nws, int nsteps)
+{
+  const bool ex = c->cfg.expansion != 0;
+  const double dt = c->cfg.dt;
+  const int stages = 2 * nws - 1;
+  for (int n = 0; n < nsteps; ++n)
+    for (int s = 0; s < stages; ++s) {
+      const double w = stage_weight(ws, nws, s);
+      // drift (aI of the stage start) + kick (half-step aI) in one pass, then the mid-stage update; the
+      // stage's first scale-factor drift rides on the previous stage's last update after the first stage
+      CHK(pass_update(c, true, true, ex, dt / 2 * w, w * dt, w * dt, ex, {{OP_PV_MID, w}}));
+      // second drift (new aI) + storeFieldsAveragesInt
+      const bool last = n == nsteps - 1 && s == stages - 1;
+      if (ex && !last)
+        CHK(pass_update(c, true, false, ex, dt / 2 * w, 0.0, 0.0, ex,
+                        {{OP_STORE_FIELDS, 0.0}, {OP_PV_SF_FIRST, stage_weight(ws, nws, (s + 1) % stages)}}));
+      else
+        CHK(pass_update(c, true, false, ex, dt / 2 * w, 0.0, 0.0, ex, {{OP_STORE_FIELDS, 0.0}}));
+    }
+  return CLMI_OK;
+}
+
+// The last resident launch, if its gate is not yet known to have opened: waits until that is decided, which the launch's
+// workgroups do when they start.  A closed gate has left the state in the arrays that were to take the final one and the
+// background in res_closed, whatever the same call queued after it: its passes (and that) run one by one now, and the
+// context goes on so.
+int settle(clmi_ctx *c)
+{
+  auto &l = c->res_last;
+  if (!l.on) return CLMI_OK;
+  l.on = false;
+  const uint32_t shut = c->res_word;
+  const auto t0 = std::chrono::steady_clock::now();
+  for (bool ended = false;;) {
+    c->res_word = __atomic_load_n(&c->res_host->word, __ATOMIC_RELAXED);
+    if (c->res_word != shut) break;
+    if (ended) return fail(c, CLMI_E_HIP, "a resident launch ended without opening or closing its gate");
+    if (std::chrono::steady_clock::now() - t0 < std::chrono::microseconds(200)) continue;
+    std::this_thread::sleep_for(std::chrono::microseconds(20));
+    const hipError_t e = hipStreamQuery(c->stream);
+    if (e != hipErrorNotReady) HIPCHK(c, e);
+    ended = e == hipSuccess;
+  }
+  if (c->res_word == shut + 1) return CLMI_OK;
+  c->resident = false;
+  c->cur_fS = l.f;
+  c->cur_pS = l.p;
+  HIPCHK(c, hipMemcpyAsync(c->dstate, c->res_closed, sizeof(DevState), hipMemcpyDeviceToDevice, c->stream));
+  switch (l.scheme) {
+    case RES_LF:
+      for (int i = 0; i < l.passes; ++i) CHK(lf_pass(c, 1.0));
+      return CLMI_OK;
+    case RES_VV:
+      return vv_passes(c, l.ws, l.nws, 0, l.passes + 1);
+    default:
+      if (!c->cfg.expansion) CHK(update(c, 0, {{OP_PV_DRIFT_AI, 0.0}}));
+      CHK(pv_passes(c, l.ws, l.nws, l.passes / 2 / (2 * l.nws - 1)));
+      return c->cfg.expansion ? CLMI_OK : update(c, 0, {});
+  }
 }
 
 // Apply the deferred drift of the last leapfrog step (drift-only pass + storeFieldsAverages).
@@ -615,7 +701,7 @@ int check_ctx(clmi_ctx *c)
 {
   if (!c) return fail(nullptr, CLMI_E_INVALID, "null context");
   HIPCHK(c, hipSetDevice(c->device));
-  return CLMI_OK;
+  return settle(c);
 }
 
 int select_arr(clmi_ctx *c, int kind, int index, int comp, DevArr **out, bool *is_field)
@@ -903,6 +989,7 @@ void clmi_destroy(clmi_ctx *c)
   if (c->done_count) (void)hipFree(c->done_count);
   if (c->res_lines) (void)hipFree(c->res_lines);
   if (c->res_gate) (void)hipFree(c->res_gate);
+  if (c->res_closed) (void)hipFree(c->res_closed);
   if (c->res_host) (void)hipHostFree(c->res_host);
   if (c->dstate) (void)hipFree(c->dstate);
   if (c->stage) (void)hipFree(c->stage);
@@ -1021,7 +1108,7 @@ int clmi_lf_evolve(clmi_ctx *c, int nsteps)
     }
     const double w = c->synced ? 0.5 : 1.0;
     if (c->pending_drift) {
-      CHK(pass_update(c, true, true, ex, dt, w * dt, w * dt, ex, {{OP_STORE_FIELDS, 0.0}, {OP_LF_MOMENTA, 0.0}}));
+      CHK(lf_pass(c, w));
     } else {
       CHK(pass_update(c, false, true, ex, 0.0, w * dt, w * dt, ex, {{OP_LF_MOMENTA, 0.0}}));
     }
@@ -1069,19 +1156,7 @@ int clmi_vv_evolve(clmi_ctx *c, const double *ws, int nws, int nsteps)
     }
     bool done = false;
     CHK(run_resident(c, RES_VV, K - 1, ws, nws, &done));
-    for (int k = done ? K - 1 : 0; k < K; ++k) {
-      const double w = wk(k);
-      if (k + 1 < K) {
-        const double w2 = wk(k + 1);
-        CHK(pass_update(c, true, true, ex, dt * w, w * dt / 2, dt / 2 * w, ex,
-                        {{OP_STORE_FIELDS, 0.0}, {OP_VV_MOMENTA, 0.0}, {OP_VV_SF_ONE, w}, {OP_VV_SF_HALF, w2},
-                         {OP_VV_MOMENTA_KICK2, 0.0}, {OP_VV_DRIFT_SF, w2}},
-                        w2 * dt / 2, dt / 2 * w2));
-      } else {
-        CHK(pass_update(c, true, true, ex, dt * w, w * dt / 2, dt / 2 * w, ex,
-                        {{OP_STORE_FIELDS, 0.0}, {OP_VV_MOMENTA, 0.0}, {OP_VV_SF_ONE, w}}));
-      }
-    }
+    CHK(vv_passes(c, ws, nws, done ? K - 1 : 0, K));
     return CLMI_OK;
   }
   for (int n = 0; n < nsteps; ++n)
@@ -1112,28 +1187,13 @@ int clmi_pv_evolve(clmi_ctx *c, const double *ws, int nws, int nsteps)
   if (!ws || nws < 1 || nsteps < 0) return fail(c, CLMI_E_INVALID, "bad composition weights");
   CHK(flush(c));
   const bool ex = c->cfg.expansion != 0;
-  const double dt = c->cfg.dt;
   const int stages = (nws - 1) * 2 + 1;
-  auto weight = [&](int s) { return ws[s < nws ? s : stages - s - 1]; };
   if (!ex) CHK(update(c, 0, {{OP_PV_DRIFT_AI, 0.0}}));
-  if (ex && nsteps > 0) CHK(update(c, 0, {{OP_PV_SF_FIRST, weight(0)}}));
+  if (ex && nsteps > 0) CHK(update(c, 0, {{OP_PV_SF_FIRST, ws[0]}}));
   bool done = false;
   if (nsteps <= INT_MAX / (2 * stages))
     CHK(run_resident(c, RES_PV, 2 * nsteps * stages, ws, nws, &done));
-  for (int n = 0; n < nsteps && !done; ++n)
-    for (int s = 0; s < stages; ++s) {
-      const double w = weight(s);
-      // drift (aI of the stage start) + kick (half-step aI) in one pass, then the mid-stage update; the
-      // stage's first scale-factor drift rides on the previous stage's last update after the first stage
-      CHK(pass_update(c, true, true, ex, dt / 2 * w, w * dt, w * dt, ex, {{OP_PV_MID, w}}));
-      // second drift (new aI) + storeFieldsAveragesInt
-      const bool last = n == nsteps - 1 && s == stages - 1;
-      if (ex && !last)
-        CHK(pass_update(c, true, false, ex, dt / 2 * w, 0.0, 0.0, ex,
-                        {{OP_STORE_FIELDS, 0.0}, {OP_PV_SF_FIRST, weight((s + 1) % stages)}}));
-      else
-        CHK(pass_update(c, true, false, ex, dt / 2 * w, 0.0, 0.0, ex, {{OP_STORE_FIELDS, 0.0}}));
-    }
+  if (!done) CHK(pv_passes(c, ws, nws, nsteps));
   // static background: restore the aSI-based drift coefficients of the other evolvers (with
   // expansion the last update already did)
   if (!ex) CHK(update(c, 0, {}));
@@ -2230,7 +2290,7 @@ int clmi_ensemble_autotune(clmi_ensemble *e, int reps, char *report, size_t repo
   if (reps < 1) reps = 1;
   EHIP(e, hipSetDevice(e->device));
   for (clmi_ctx *c : e->m)
-    if (sync_stream(c) != CLMI_OK) return efail(e, CLMI_E_HIP, "member: " + c->err);
+    if (settle(c) != CLMI_OK || sync_stream(c) != CLMI_OK) return efail(e, CLMI_E_HIP, "member: " + c->err);
   CHK(ens_tables(e));
   hipEvent_t t0 = nullptr, t1 = nullptr;
   EHIP(e, hipEventCreate(&t0));
@@ -2322,7 +2382,7 @@ int clmi_ensemble_lf_evolve(clmi_ensemble *e, int nsteps)
     --nsteps;
   }
   for (clmi_ctx *c : e->m)
-    if (sync_stream(c) != CLMI_OK) return efail(e, CLMI_E_HIP, "member: " + c->err);
+    if (settle(c) != CLMI_OK || sync_stream(c) != CLMI_OK) return efail(e, CLMI_E_HIP, "member: " + c->err);
   CHK(ens_tables(e));
   // two steps (both buffer parities) of every group per graph replay
   if (nsteps >= 2 && !e->exec) CHK(ens_capture(e));

@@ -284,6 +284,7 @@ struct ResidentArgs {
   int refuse;          // the gate stays shut (testing)
   ResidentGate *gate;
   ResidentHost *host;
+  DevState *closed_st; // takes *st where the gate closes
   uint32_t arrived;    // workgroups that have arrived at the gate once all of this launch have
   uint32_t shut;       // the gate's word before this launch; shut + 1: open, shut + 2: closed for good
 };

@@ -25,8 +25,8 @@
 // The launch is cooperative, but that check knows nothing of what else holds the device's CUs (another process's
 // launch of this kind may wait for ours), so a workgroup first arrives at a gate.  The last to arrive opens it; one
 // that waits there for kGateLimit polls (about a second) closes it, whichever comes first, and the host learns which.
-// Nothing is written before the gate, so a closed one costs the wait alone: the host runs the same passes one by
-// one.  Behind an open gate every workgroup is on the chip and every wait ends; kSpinLimit is there so that
+// Behind a closed one every workgroup stores the state as it loaded it, so that what the host has queued meanwhile finds
+// a state in the arrays that take it; the host then runs the same passes one by one.  Behind an open gate every workgroup is on the chip and every wait ends; kSpinLimit is there so that
 // the grid drains even if the device itself fails, and the state is lost then (the host reports it).
 //
 // Measured (MI355X, us per leapfrog pass, resident against pass and update launches; VV2 in brackets):
@@ -391,8 +391,35 @@ __global__ __launch_bounds__(kResThreads) void k_scalar_resident(const ResidentA
     }
   }
   if (tid == 0) dead = !pass_gate(r);
+  auto store_state = [&]() {
+    if (act)
+#pragma unroll
+      for (int f = 0; f < NF; ++f)
+#pragma unroll
+        for (int p = 0; p < P; ++p)
+          if (has(p)) {
+            const uint32_t s = slot(p) + own;
+            vstore<VZ, false>((M *)a.pi_out[f], s, pi[p][f]);
+            if constexpr (!F32) {
+              vstore<VZ, false>((double *)a.phi_out[f], s, phi[p][f]);
+            } else {
+              float h[VZ], l[VZ];
+#pragma unroll
+              for (int k = 0; k < VZ; ++k) {
+                h[k] = phi[p][f][k].x;
+                l[k] = phi[p][f][k].y;
+              }
+              vstore<VZ, false>((float *)a.phi_out[f], s, h);
+              vstore<VZ, false>(a.philo_out[f], s, l);
+            }
+          }
+  };
   __syncthreads();
-  if (dead) return;
+  if (dead) {
+    store_state();
+    if (blockIdx.x == 0 && tid == 0) *r.closed_st = S;
+    return;
+  }
 
   const bool red = r.mc.expansion != 0;
   const double dt = r.mc.dt;
@@ -666,27 +693,7 @@ __global__ __launch_bounds__(kResThreads) void k_scalar_resident(const ResidentA
   }
   if (!ok) return;
 
-  if (act)
-#pragma unroll
-    for (int f = 0; f < NF; ++f)
-#pragma unroll
-      for (int p = 0; p < P; ++p)
-        if (has(p)) {
-          const uint32_t s = slot(p) + own;
-          vstore<VZ, false>((M *)a.pi_out[f], s, pi[p][f]);
-          if constexpr (!F32) {
-            vstore<VZ, false>((double *)a.phi_out[f], s, phi[p][f]);
-          } else {
-            float h[VZ], l[VZ];
-#pragma unroll
-            for (int k = 0; k < VZ; ++k) {
-              h[k] = phi[p][f][k].x;
-              l[k] = phi[p][f][k].y;
-            }
-            vstore<VZ, false>((float *)a.phi_out[f], s, h);
-            vstore<VZ, false>(a.philo_out[f], s, l);
-          }
-        }
+  store_state();
   if (red && blockIdx.x == 0 && tid == 0) *r.st = S;
 }
 

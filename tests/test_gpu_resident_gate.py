@@ -1,6 +1,6 @@
-"""GPU: the gate of the resident evolver.  Its workgroups write nothing until all have started; where they cannot, the
-gate closes, the call takes its passes one by one and the context goes on that way, with the same bits.
-CLMI_FLAG_REFUSE_RESIDENT keeps the gate shut from the host."""
+"""GPU: the gate of the resident evolver.  Its workgroups evolve nothing until all have started; where they cannot, the
+gate closes, the state passes through unchanged, and the context's next call takes the passes one by one, as all later
+ones do, with the same bits.  CLMI_FLAG_REFUSE_RESIDENT keeps the gate shut from the host."""
 import numpy as np
 import pytest
 
@@ -38,14 +38,15 @@ def test_closed_gate_leaves_the_passes(gpu, N, prec, scheme, expansion):
     for flags in (0, CLMI_FLAG_REFUSE_RESIDENT):
         lat = start(N, prec, expansion, flags)
         assert "k_scalar_resident" in lat.plan()
-        for n in (7, 5, 9):  # the first of them meets the gate
+        for n in (7, 5, 9):  # the first of them meets the gate; the whole state must be what its passes leave
             if scheme == "LF":
                 lat.lf_evolve(n)
             elif scheme == "VV2":
                 lat.vv_evolve(VV_WEIGHTS[scheme], n)
             else:
                 lat.pv_evolve(PV_WEIGHTS[scheme], n)
-            # an open gate keeps the evolver in use, a closed one ends it
+            # an open gate keeps the evolver in use, a closed one ends it (at the context's next call)
+            lat.synchronize()
             assert ("k_scalar_resident" in lat.plan()) == (flags == 0)
         if scheme == "LF":
             lat.lf_sync()
