@@ -113,8 +113,10 @@ template <bool F32, bool NT> __device__ __forceinline__ void store_v(void *f, fl
 // same fields, so one pass does both and keeps the sums after each.  It is the drift + kick pass plus a few operations,
 // where the second pass moved the whole state again.  A velocity-Verlet step, two passes / one (us, FP64 and FP32-bulk):
 // 64^3 51.1 / 30.5 and 44.8 / 25.6, 100^3 138 / 83 and 112 / 63, 128^3 182 / 120 and 116 / 63, 200^3 815 / 539 and
-// 657 / 399, 256^3 1252 / 862 and 853 / 484.  FP64 asks for two waves a SIMD: left alone it takes two registers more
-// than they have.
+// 657 / 399, 256^3 1252 / 862 and 853 / 484.  FP64 asks for two waves a SIMD (left alone it takes two registers more
+// than they have) and spills 8 registers for them (36 bytes of scratch a lane; 6 and 28 on ragged tiles), which is why its
+// second kick costs 30 %.  In FP32-bulk it costs its instructions: 199 registers with one kick, 207 with two, and vector units
+// that are busy 75 % of the time with either.
 template <bool F32, bool DRIFT, bool KICK, bool RED, int GTY, int U1 = 0, bool RAG = false, bool NT = !RAG, bool KICK2 = false>
 __global__ __launch_bounds__(64 * GTY, KICK2 && !F32 ? 2 : 1) void k_gauge_tiled(const GaugePassArgs a, const int XC, const int RG)
 {

@@ -12,8 +12,8 @@ hipError_t launch_scalar_flat_f32_nf1(bool drift, bool kick, bool red, const Sca
 hipError_t launch_scalar_flat_f32_nf2(bool drift, bool kick, bool red, const ScalarPassArgs &a, const FlatPlan &p,
                                       hipStream_t s, bool kick2);
 
-// Even N from 24 (below, a lattice has fewer sites than a few workgroups' chunks) to 500 (two LDS rows of two fields
-// in 64 KiB).  One site per lane up to N = 64, two above; the resident evolver's groups up to N = 128.  The x-chunk
+// Even N from 24 (below, a lattice has fewer sites than a few workgroups' chunks) to 500, the largest measured (two
+// fields: 66 168 bytes of LDS with the pass's tail, two workgroups a CU; the halo is two pairs a thread up to 512).  One site per lane up to N = 64, two above; the resident evolver's groups up to N = 128.  The x-chunk
 // is one group: many short marches balance the CUs and keep the x-halo in L2 (us a step, two fields FP64, x-chunk 8
 // / 16 / 24 / 32: 180^3 92 / 96 / 88 / 99, 200^3 119 / 140 / 138 / 158, 250^3 226 / 229 / 250 / 230; 300^3 from 16:
 // 386 / - / 400).
