@@ -520,8 +520,8 @@ constexpr int kResMinPasses = 4;
 // drift + kick passes (RES_LF), double-kick passes (RES_VV) or pairs of drift + kick and drift (RES_PV).
 // *done = false: not taken (nothing was changed), the caller runs the passes one by one, which gives the
 // same bits.  Not taken: too few passes for the cooperative launch to pay, pass timing on, a background snapshot
-// asked for, more weights than its arguments hold, no memory for its buffers, or a launch that the device refuses (after
-// which the context does not try again).  Whether the launch's gate opened is found out by the context's next call
+// asked for, more weights than its arguments hold, no memory for its buffers, or a launch that the runtime refuses, as it
+// does in every process of a card but the first that makes one (after which the context does not try again).  Whether the launch's gate opened is found out by the context's next call
 // (settle), so that calls on several contexts still queue their work without waiting for one another.
 int run_resident(clmi_ctx *c, int scheme, int passes, const double *ws, int nws, bool *done)
 {
