@@ -16,7 +16,13 @@ def test_first_resident_call_takes_little_memory(gpu, prec, nf):
 
     say(f"case resident memory prec={prec} nf={nf}")
     N = 128
-    lat = Lattice(lphi4(100.0, n_fields=nf, phi0_gev=5.6964e18, lam=1.0, pi0_program=-0.5), N, 0.4909, 0.005, prec)
+    spec = lphi4(100.0, n_fields=nf, phi0_gev=5.6964e18, lam=1.0, pi0_program=-0.5)
+    # the process's first cooperative launch makes the runtime allocate its queue for them
+    first = Lattice(spec, 32, 0.4909, 0.005, prec)
+    first.lf_init()
+    first.lf_evolve(8)
+    first.synchronize()
+    lat = Lattice(spec, N, 0.4909, 0.005, prec)
     for k in (FLD_S, PI_S):
         for f in range(nf):
             lat.upload(k, f, 0, 0.3 * np.random.default_rng(f).standard_normal((N, N, N)))
@@ -34,3 +40,4 @@ def test_first_resident_call_takes_little_memory(gpu, prec, nf):
     # a momentum array is 8 or 16 MiB; a few small allocations share at most two blocks of 2 MiB
     assert free - torch.cuda.mem_get_info()[0] < 5 << 20
     lat.close()
+    first.close()
